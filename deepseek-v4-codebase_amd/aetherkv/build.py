@@ -61,7 +61,7 @@ def sources():
     return sorted(list(CSRC.glob("*.hip")) + list(CSRC.glob("*.cpp")))
 
 
-# Per-source flags.  quant_attn_mfma.hip, sink_attention_mfma.hip: the split combines' scalar
+# Per-source flags.  quant_attn_mfma.hip, sink_attention_mfma.hip, sink_attention_f32.hip: the split combines' scalar
 # arguments arrive in registers at dispatch (their one memory round then does not wait for the
 # argument block; byval struct arguments, as the other kernels there take, are not preloaded).
 # Measured per kernel: it helps the combine (HCA decode) and left the codec kernels within noise or
@@ -70,6 +70,7 @@ _PRELOAD = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
 SOURCE_FLAGS = {
     "quant_attn_mfma.hip": _PRELOAD,
     "sink_attention_mfma.hip": _PRELOAD,
+    "sink_attention_f32.hip": _PRELOAD,
 }
 
 

@@ -58,6 +58,14 @@ size_t sink_attention_mfma_workspace(bool dense, int64_t B, int64_t T, int64_t H
 int sink_attention_mfma(const void* q, const void* kv, const void* idx, int idx_kind, const void* sink,
                         int sink_scalar, int32_t dtype, int64_t B, int64_t T, int64_t H, int64_t S, int64_t K,
                         float scale, void* ws, size_t ws_bytes, void* out, hipStream_t st, const char* who);
+// The same in fp32 arithmetic (sink_attention_f32.hip): fp32 at head_dim 64 / 128, 16-bit at 64; q, kv and
+// out aligned to four elements.  A workspace that is too small or misaligned runs the call unsplit.
+bool sink_attention_f32_supported(int32_t dtype, int64_t D);
+bool sink_attention_f32_fits(bool dense, int64_t D, int64_t B, int64_t T, int64_t H, int64_t S, int64_t K);
+size_t sink_attention_f32_workspace(bool dense, int64_t D, int64_t B, int64_t T, int64_t H, int64_t K);
+int sink_attention_f32(const void* q, const void* kv, const void* idx, int idx_kind, const void* sink, int sink_scalar,
+                       int32_t dtype, int64_t B, int64_t T, int64_t H, int64_t D, int64_t S, int64_t K, float scale,
+                       void* ws, size_t ws_bytes, void* out, hipStream_t st, const char* who);
 // The flash kernel for dense calls (prefill_flash.hip): 64 (target, head) rows per workgroup, tiles
 // of dense_flash_tile() sources; with n_split > 1 each row's tiles are split into n_split pieces
 // whose (max, sum, O) go to part (the layout of sink_attention_mfma's combine).

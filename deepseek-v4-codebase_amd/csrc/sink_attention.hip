@@ -4,8 +4,9 @@
 //    semantics aether_kernels/csrc/sparse_sink_attention_cuda.cu:47-114, oracle
 //    aether_pipeline/serving.py:99-130) and, with dense indices, for tiled_prefill_attention
 //    (aether_kernels/sparse_attention.py:19-42) with the sink counted once as in
-//    aether_2b/modeling.py:158-178, for fp32 inputs and head dims other than 128 (bf16/fp16 at
-//    head_dim 128 run on the matrix cores, sink_attention_mfma.hip).  One wave per (b, t, h); keys
+//    aether_2b/modeling.py:158-178, for head dims other than 64 and 128 and for misaligned
+//    tensors (the others run on the matrix cores, sink_attention_mfma.hip and
+//    sink_attention_f32.hip).  One wave per (b, t, h); keys
 //    streamed in tiles of 64 with an online softmax; the sink joins the normaliser once at the end.
 // 2. quant_attn_partial_kernel + quant_attn_combine_kernel — one decode token per row over
 //    TurboQuant-compressed shared K=V blocks (selected by the CSA indexer, or all blocks for HCA)
@@ -372,6 +373,11 @@ int sparse_common(const void* q, const void* kv, const void* topk, int idx_kind,
       (K == 0 || is_aligned(kv, 16)) && is_aligned(sink, 2))
     return sink_attention_mfma(q, kv, topk, idx_kind, sink, scalar, dtype, B, T, H, S, K, scale, ws, ws_bytes, out, st,
                                who);
+  const size_t quad = 4 * dtype_size(dtype);
+  if (sink_attention_f32_supported(dtype, D) && sink_attention_f32_fits(idx_kind == 0, D, B, T, H, S, K) &&
+      is_aligned(q, quad) && is_aligned(out, quad) && (K == 0 || is_aligned(kv, quad)))
+    return sink_attention_f32(q, kv, topk, idx_kind, sink, scalar, dtype, B, T, H, D, S, K, scale, ws, ws_bytes, out,
+                              st, who);
   if (dtype == AEKV_F32) launch_sparse<AEKV_F32>(idx_kind, q, kv, topk, sink, scalar, B, T, H, D, S, K, scale, out, st);
   else if (dtype == AEKV_F16) launch_sparse<AEKV_F16>(idx_kind, q, kv, topk, sink, scalar, B, T, H, D, S, K, scale, out, st);
   else launch_sparse<AEKV_BF16>(idx_kind, q, kv, topk, sink, scalar, B, T, H, D, S, K, scale, out, st);
@@ -436,7 +442,12 @@ extern "C" int aekv_tiled_prefill_attention(const void* q, const void* kv, const
 
 extern "C" size_t aekv_sink_attention_workspace_size(int32_t dtype, int64_t B, int64_t T, int64_t H, int64_t D,
                                                      int64_t S, int64_t K) {
-  if (!sink_attention_mfma_supported(dtype, D) || B <= 0 || T <= 0 || H <= 0 || S < 0) return 0;
+  if (!is_float_dtype(dtype) || B <= 0 || T <= 0 || H <= 0 || S < 0) return 0;
+  if (sink_attention_f32_supported(dtype, D)) {
+    const int64_t n = K < 0 ? S : K;
+    return sink_attention_f32_fits(K < 0, D, B, T, H, S, n) ? sink_attention_f32_workspace(K < 0, D, B, T, H, n) : 0;
+  }
+  if (!sink_attention_mfma_supported(dtype, D)) return 0;
   return K < 0 ? sink_attention_mfma_workspace(true, B, T, H, S, S) : sink_attention_mfma_workspace(false, B, T, H, S, K);
 }
 

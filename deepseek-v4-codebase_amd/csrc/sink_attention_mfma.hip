@@ -25,7 +25,7 @@
 // ratios carry one rounding each (2^-9 relative in bf16, 2^-12 in fp16).
 #include <algorithm>
 
-#include "aekv_common.h"
+#include "sink_combine.h"
 
 namespace aekv {
 namespace {
@@ -33,9 +33,9 @@ namespace {
 constexpr int kD = 128;
 constexpr int kGroup = 32;            // sources per wave step
 constexpr int kObStride = kD + 4;     // merge rows: head h at bank 4h (no conflicts)
-constexpr int kPartStride = kD + 4;   // one piece of one (target, head): max, sum, 2 pad, O[128]
-constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kNegInf = -__builtin_inff();
+constexpr int kPartStride = sinkc::kPartStride<kD>;  // one piece of one (target, head)
+using sinkc::kLog2e;
+using sinkc::kNegInf;
 
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
@@ -268,74 +268,6 @@ __global__ __launch_bounds__(64 * NW) void gather_attn_kernel(GatherArgs a) {
   }
 }
 
-// Merges the source pieces of each (target, head) row: M = max(sink, piece maxima),
-// L = 2^(sink - M) + sum_p 2^(m_p - M) l_p, out = sum_p 2^(m_p - M) O_p / L (log2 units), as an
-// online merge over chunks of 8 pieces whose loads are all issued together.  32 threads per row,
-// 4 dims each, NT / 32 rows per workgroup: 8, or 2 when 8 would leave CUs without a workgroup, so
-// that a call of few rows spreads its loads over as many CUs.
-template <int DT, int NT>
-__global__ __launch_bounds__(NT) void sink_attn_combine_kernel(const float* __restrict__ part, int n_split,
-                                                               const uint16_t* __restrict__ sink, int sink_scalar,
-                                                               int H, int rows, uint16_t* __restrict__ out) {
-  using E = Elem<DT>;
-  constexpr int kChunk = 8;
-  const int row = static_cast<int>(blockIdx.x) * (NT / 32) + (static_cast<int>(threadIdx.x) >> 5);
-  if (row >= rows) return;
-  const int j = threadIdx.x & 31;
-  const float* p = part + static_cast<int64_t>(row) * n_split * kPartStride;
-  float m[kChunk], l[kChunk];
-  f32x4_t o[kChunk];
-  // A chunk's loads (and the sink's, with the first) all precede the empty asm that takes their
-  // values, so every load is issued before the first wait (the compiler would otherwise wait for
-  // the sink first, and move loads into the branches that use them, each with its own wait).  A
-  // piece past n_split reads piece 0 and is replaced by the empty state.
-  auto load_chunk = [&](const int s0, uint32_t* skb) {
-    float2 ml[kChunk];
-#pragma unroll
-    for (int i = 0; i < kChunk; ++i) {
-      const float* ps = p + (s0 + i < n_split ? s0 + i : 0) * kPartStride;
-      ml[i] = *reinterpret_cast<const float2*>(ps);
-      o[i] = *reinterpret_cast<const f32x4_t*>(ps + 4 + 4 * j);
-    }
-    if (skb) *skb = sink[sink_scalar ? 0 : row % H];
-#pragma unroll
-    for (int i = 0; i < kChunk; ++i) asm volatile("" : "+v"(ml[i].x), "+v"(ml[i].y), "+v"(o[i]));
-    if (skb) asm volatile("" : "+v"(*skb));
-#pragma unroll
-    for (int i = 0; i < kChunk; ++i) {
-      const bool in = s0 + i < n_split;
-      m[i] = in ? ml[i].x : kNegInf;
-      l[i] = in ? ml[i].y : 0.0f;
-      o[i] = in ? o[i] : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    }
-  };
-  uint32_t skb;
-  load_chunk(0, &skb);
-  const float sk = E::to_f32(skb) * kLog2e;
-  float M = sk, den = sk == kNegInf ? 0.0f : 1.0f;
-  f32x4_t acc = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  for (int s0 = 0; s0 < n_split; s0 += kChunk) {
-    if (s0 > 0) load_chunk(s0, nullptr);
-    float cm = M;
-#pragma unroll
-    for (int i = 0; i < kChunk; ++i) cm = fmaxf(cm, m[i]);
-    if (cm == kNegInf) continue;  // nothing yet (no sink, no source)
-    const float r = M == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(M - cm);
-    den *= r;
-    acc *= r;
-    M = cm;
-#pragma unroll
-    for (int i = 0; i < kChunk; ++i) {
-      const float f = m[i] == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(m[i] - M);
-      den = fmaf(f, l[i], den);
-      acc = f32x4_t{fmaf(f, o[i][0], acc[0]), fmaf(f, o[i][1], acc[1]), fmaf(f, o[i][2], acc[2]), fmaf(f, o[i][3], acc[3])};
-    }
-  }
-  const float r = den > 0.0f ? 1.0f / den : 0.0f;
-  *reinterpret_cast<uint2*>(out + static_cast<int64_t>(row) * kD + 4 * j) =
-      make_uint2(E::pack(acc[0] * r, acc[1] * r), E::pack(acc[2] * r, acc[3] * r));
-}
-
 template <int DT, int IDX>
 void launch_gather_t(const GatherArgs& a, int64_t rows, int hgroups, int nw, hipStream_t st) {
   const dim3 grid(static_cast<uint32_t>(rows), static_cast<uint32_t>(hgroups), static_cast<uint32_t>(a.n_split));
@@ -439,23 +371,11 @@ int sink_attention_mfma(const void* q, const void* kv, const void* idx, int idx_
   }
   if (p.n_split == 1) return AEKV_OK;
   const int64_t n = rows * H;
-  const int nt = ceil_div(n, int64_t(8)) >= 256 ? 256 : 64;
-  const int64_t n_wg = ceil_div(n, static_cast<int64_t>(nt / 32));
   if (n > 0x7fffffffLL) return fail(AEKV_ERR_UNSUPPORTED, "%s: too many rows", who);
-  const dim3 grid(static_cast<uint32_t>(n_wg));
-  const uint16_t* sk = static_cast<const uint16_t*>(sink);
-  uint16_t* o = static_cast<uint16_t*>(out);
-  const int hh = static_cast<int>(H);
-  auto launch = [&](auto kern) {
-    hipLaunchKernelGGL(kern, grid, dim3(nt), 0, st, part, p.n_split, sk, sink_scalar, hh, static_cast<int>(n), o);
-  };
-  if (dtype == AEKV_BF16) {
-    if (nt == 256) launch(sink_attn_combine_kernel<AEKV_BF16, 256>);
-    else launch(sink_attn_combine_kernel<AEKV_BF16, 64>);
-  } else {
-    if (nt == 256) launch(sink_attn_combine_kernel<AEKV_F16, 256>);
-    else launch(sink_attn_combine_kernel<AEKV_F16, 64>);
-  }
+  if (dtype == AEKV_BF16)
+    sinkc::launch_combine<AEKV_BF16, kD>(part, p.n_split, sink, sink_scalar, static_cast<int>(H), n, out, st);
+  else
+    sinkc::launch_combine<AEKV_F16, kD>(part, p.n_split, sink, sink_scalar, static_cast<int>(H), n, out, st);
   return check_launch(who);
 }
 

@@ -174,8 +174,9 @@ int aekv_sparse_sink_attention(const void* q, const void* kv, const void* topk, 
                                float softmax_scale, void* out, void* stream);
 
 /* The same, with a caller-owned workspace (the binding's own allocation in the reference,
- * bindings.cpp:21-46, happens in the caller here): bf16/fp16 calls at D = 128 whose launch would
- * leave most CUs idle split each target's sources over several workgroups and merge the pieces.
+ * bindings.cpp:21-46, happens in the caller here): calls at D = 128 or 64 whose launch would
+ * leave most CUs idle split each target's sources over several workgroups and merge the pieces
+ * (fp32 calls, and 16-bit ones at D = 64, run unsplit when the workspace is too small).
  * ws_bytes from aekv_sink_attention_workspace_size(dtype, B, T, H, D, S, K); ws = NULL runs unsplit
  * (the entry point above); a non-NULL ws must be 256-byte aligned and large enough. */
 int aekv_sparse_sink_attention_ws(const void* q, const void* kv, const void* topk, int32_t idx_dtype,
