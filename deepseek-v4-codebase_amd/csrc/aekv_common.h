@@ -33,6 +33,11 @@ size_t mfma_indexer_workspace(int64_t B, int64_t S, int32_t k);
 int launch_mfma_indexer(const float* q, const float* w, const void* codes, const float* kscale, const float* diag,
                         const int32_t* valid, int64_t B, int64_t T, int64_t S, int IH, int IC, int bits, int k,
                         int mode, void* ws, int64_t* out_idx, float* out_score, hipStream_t st, const char* who);
+// The same over fp32 keys [B, S, IC], under the same limits (csa_indexer_f32.hip); q and keys 16-byte
+// aligned, the workspace mfma_indexer_workspace's.
+int launch_f32_indexer(const float* q, const float* w, const float* keys, const int32_t* valid, int64_t B, int64_t S,
+                       int IH, int IC, int k, int mode, void* ws, int64_t* out_idx, float* out_score, hipStream_t st,
+                       const char* who);
 bool use_specialised_codec();
 // Host-side argument checks of the quantised-key indexer for B * T rows (csa_indexer.hip).
 int validate_quant_rows(const float* index_q, const float* index_weight, const void* key_codes,

@@ -389,6 +389,9 @@ extern "C" int aekv_csa_indexer_topk(const float* index_q, const float* index_kv
   if (int rc = validate_common(index_q, index_weight, B, S, IH, IC, k, mode, ws, ws_bytes, out_idx, who)) return rc;
   if (B == 0) return AEKV_OK;
   if (S > 0 && !index_kv) return fail(AEKV_ERR_VALUE, "%s: null index_kv", who);
+  if (use_specialised_codec() && mfma_indexer_supported(IH, IC, k, S) && is_aligned(index_q, 16) && is_aligned(index_kv, 16))
+    return launch_f32_indexer(index_q, index_weight, index_kv, valid, B, S, IH, IC, k, mode, ws, out_idx, out_score,
+                              as_stream(stream), who);
   IndexerArgs a{};
   a.q = index_q;
   a.w = index_weight;

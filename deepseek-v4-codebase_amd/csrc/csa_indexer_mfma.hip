@@ -40,12 +40,7 @@ int launch_mfma_score(MfmaIdxArgs& a, const float* q, const float* w, const void
   a.k = k;
   a.mode = mode;
   a.wscale = wht_scale(IC);
-  const WsLayout l = layout(B, S);
-  char* base = static_cast<char*>(ws);
-  a.keys = reinterpret_cast<uint32_t*>(base + l.keys);
-  a.smax = reinterpret_cast<uint32_t*>(base + l.smax);
-  a.ms = static_cast<int64_t>(align_up((static_cast<size_t>(S) + 15) / 16, 4));
-  a.ks = static_cast<int64_t>(align_up(static_cast<size_t>(S), 16));
+  bind_workspace(a, B, S, ws);
 
   const int nrb = (IH + 3) / 4;
   // prefill rows (T > 1 targets per key row) share each key group kScoreTT rows at a time
@@ -72,6 +67,31 @@ int launch_mfma_score(MfmaIdxArgs& a, const float* q, const float* w, const void
   return check_launch(who);
 }
 
+void bind_workspace(MfmaIdxArgs& a, int64_t B, int64_t S, void* ws) {
+  const WsLayout l = layout(B, S);
+  char* base = static_cast<char*>(ws);
+  a.S = S;
+  a.keys = reinterpret_cast<uint32_t*>(base + l.keys);
+  a.smax = reinterpret_cast<uint32_t*>(base + l.smax);
+  a.ms = static_cast<int64_t>(align_up((static_cast<size_t>(S) + 15) / 16, 4));
+  a.ks = static_cast<int64_t>(align_up(static_cast<size_t>(S), 16));
+}
+
+int launch_select(const MfmaIdxArgs& a, int64_t B, int64_t* out_idx, float* out_score, hipStream_t st, const char* who) {
+  const uint32_t by = static_cast<uint32_t>(B);
+  // rows of at most 16384 keys load 2 (512 threads) or 1 (1024 threads) slot columns per thread
+  const bool few_slots = slot_cols_fit(a.S, 512, 2);
+  if (B >= 1024 && a.k <= 512) {
+    auto fn = few_slots ? idx_mfma_final_kernel<512, 1536, 2> : idx_mfma_final_kernel<512, 1536, kHistBins / 512>;
+    hipLaunchKernelGGL(fn, dim3(by), dim3(512), 0, st, a, out_idx, out_score);
+  } else {
+    auto fn = few_slots ? idx_mfma_final_kernel<kSelThreads, kCandCap, 1>
+                        : idx_mfma_final_kernel<kSelThreads, kCandCap, kHistBins / kSelThreads>;
+    hipLaunchKernelGGL(fn, dim3(by), dim3(kSelThreads), 0, st, a, out_idx, out_score);
+  }
+  return check_launch(who);
+}
+
 }  // namespace idx
 
 using namespace idx;
@@ -93,18 +113,7 @@ int launch_mfma_indexer(const float* q, const float* w, const void* codes, const
   MfmaIdxArgs a{};
   if (int rc = launch_mfma_score(a, q, w, codes, kscale, diag, valid, B, T, S, IH, IC, bits, k, mode, ws, st, who))
     return rc;
-  const uint32_t by = static_cast<uint32_t>(B);
-  // rows of at most 16384 keys load 2 (512 threads) or 1 (1024 threads) slot columns per thread
-  const bool few_slots = slot_cols_fit(S, 512, 2);
-  if (B >= 1024 && k <= 512) {
-    auto fn = few_slots ? idx_mfma_final_kernel<512, 1536, 2> : idx_mfma_final_kernel<512, 1536, kHistBins / 512>;
-    hipLaunchKernelGGL(fn, dim3(by), dim3(512), 0, st, a, out_idx, out_score);
-  } else {
-    auto fn = few_slots ? idx_mfma_final_kernel<kSelThreads, kCandCap, 1>
-                        : idx_mfma_final_kernel<kSelThreads, kCandCap, kHistBins / kSelThreads>;
-    hipLaunchKernelGGL(fn, dim3(by), dim3(kSelThreads), 0, st, a, out_idx, out_score);
-  }
-  return check_launch(who);
+  return launch_select(a, B, out_idx, out_score, st, who);
 }
 
 }  // namespace aekv

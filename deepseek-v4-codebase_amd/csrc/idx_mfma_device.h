@@ -63,6 +63,7 @@ __host__ __device__ constexpr int score_spw(int bits, int ic, int tt) {
 }
 
 typedef __attribute__((ext_vector_type(4))) int i32x4_t;
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
 
 __device__ __forceinline__ float softplus_f32(float x) { return x > 20.0f ? x : log1pf(expf(x)); }
 
@@ -1066,6 +1067,29 @@ __device__ __forceinline__ uint32_t select_row(const MfmaIdxArgs& a, const int b
   }
 
   // ---- 2. three radix levels down to the kk-th largest key T ----
+  // Passes over all of the row's stored keys (candidates that overflow LDS), four adjacent keys per
+  // lane: vector v holds keys 4 v .. 4 v + 3 (those at or past the count are not the row's).  f(key,
+  // index, in) is called by whole waves.
+  const int nv_i = static_cast<int>(nv), n_vec = (nv_i + 3) >> 2;
+  auto load_vec = [&](int v) {
+    return static_cast<u32x4_t>(__builtin_amdgcn_raw_buffer_load_b128(krs, static_cast<uint32_t>(v) * 16u, 0, 0));
+  };
+  auto for_part_keys = [&](int v0, int v1, auto&& f) {  // this wave alone
+#pragma unroll 1
+    for (int v = v0; v < v1; v += 64) {
+      const u32x4_t kw = load_vec(v + lane);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) f(kw[e], 4 * (v + lane) + e, 4 * (v + lane) + e < nv_i && v + lane < v1);
+    }
+  };
+  auto for_all_keys = [&](int v0, int v1, auto&& f) {  // every wave its share of the workgroup's steps
+#pragma unroll 1
+    for (int v = v0 + 64 * wv; v < v1; v += NT) {
+      const u32x4_t kw = load_vec(v + lane);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) f(kw[e], 4 * (v + lane) + e, 4 * (v + lane) + e < nv_i);
+    }
+  };
   uint32_t need = kk;  // keys still to take at or below the current prefix
   uint32_t prefix = 0u;
   int shift = 32;
@@ -1085,10 +1109,19 @@ __device__ __forceinline__ uint32_t select_row(const MfmaIdxArgs& a, const int b
         if (lvl == 0 || (key >> shift) == prefix) atomicAdd(&h[(key >> nshift) & mask], 1u);
       }
     } else {
-      for (int64_t j = tid; j < nv; j += NT) {
-        const uint32_t key = krow[j];
-        if (lvl == 0 || (key >> shift) == prefix) atomicAdd(&h[(key >> nshift) & mask], 1u);
-      }
+      // Rows come here because many keys are equal, so lanes of a wave mostly meet in one bin: the
+      // bin of the wave's first counted key takes one atomic for all of its lanes there.
+      for_all_keys(0, n_vec, [&](const uint32_t key, const int, const bool in) {
+        const bool act = in && (lvl == 0 || (key >> shift) == prefix);
+        const uint64_t am = __builtin_amdgcn_ballot_w64(act);
+        if (am == 0u) return;  // wave-uniform
+        const uint32_t bin = (key >> nshift) & mask;
+        const int first = __builtin_ctzll(am);
+        const uint32_t b0 = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(bin), first));
+        const uint64_t same = __builtin_amdgcn_ballot_w64(act && bin == b0);
+        if (lane == first) atomicAdd(&h[b0], static_cast<uint32_t>(__builtin_popcountll(same)));
+        if (act && bin != b0) atomicAdd(&h[bin], 1u);
+      });
     }
     __syncthreads();
     uint32_t t, ab, ct;
@@ -1114,49 +1147,58 @@ __device__ __forceinline__ uint32_t select_row(const MfmaIdxArgs& a, const int b
     s_cnt[1] = 0u;
   }
   __syncthreads();
-  if (fast) {
-    const bool all_eq = n_eq == need;
+  if (fast && n_eq == need) {  // every key == T is taken: any order
     for (int i = tid; i < n; i += NT) {
       const uint32_t key = ck[i], idx = ci[i];
       const uint32_t pg = wave_reserve<1>(&s_cnt[0], key > T ? 1u : 0u);
-      const uint32_t pe = wave_reserve<1>(&s_cnt[1], key == T && all_eq ? 1u : 0u);
+      const uint32_t pe = wave_reserve<1>(&s_cnt[1], key == T ? 1u : 0u);
       if (key > T) {
         if (pg < n_gt) sel[pg] = sort_word(key, idx);
       } else if (key == T) {
-        if (all_eq) {
-          if (pe < need) sel[n_gt + pe] = sort_word(key, idx);
-        } else {  // ties at T: rank among the equal keys by index
-          uint32_t r = 0;
-          for (int j = 0; j < n; ++j) r += (ck[j] == T && ci[j] < idx) ? 1u : 0u;
-          if (r < need) sel[n_gt + r] = sort_word(key, idx);
-        }
+        if (pe < need) sel[n_gt + pe] = sort_word(key, idx);
       }
     }
   } else {
-    uint32_t eq_run = 0;
-    for (int64_t base = 0; base < nv; base += NT) {
-      const int64_t j = base + tid;
-      const uint32_t key = j < nv ? krow[j] : 0u;
-      const bool gt = j < nv && key > T;
-      const bool eq = j < nv && key == T;
+    // Wave w takes the w-th contiguous part of the row.  First pass: keys > T are placed (in any
+    // order) and the part's keys == T counted; second pass: keys == T are placed in index order,
+    // after those of the waves before, until `need` of them are.  No barrier inside either pass.
+    // (Also for collected candidates with more keys == T than are taken: ranking those by index among
+    // themselves compared every pair, 660 us for the 4096 zero scores of a 65536-key row.)
+    const int per = (n_vec + NW * 64 - 1) / (NW * 64) * 64;  // whole wave steps
+    const int v0 = wv * per, v1 = min(n_vec, v0 + per);
+    uint32_t eq = 0u;  // wave-uniform
+    for_part_keys(v0, v1, [&](const uint32_t key, const int j, const bool in) {
+      const bool gt = in && key > T;
+      eq += static_cast<uint32_t>(__builtin_popcountll(__builtin_amdgcn_ballot_w64(in && key == T)));
+      if (__builtin_amdgcn_ballot_w64(gt) == 0u) return;  // wave-uniform
       const uint32_t pg = wave_reserve<1>(&s_cnt[0], gt ? 1u : 0u);
       if (gt && pg < n_gt) sel[pg] = sort_word(key, static_cast<uint32_t>(j));
-      const uint64_t m = __builtin_amdgcn_ballot_w64(eq);
-      if (lane == 0) s_wave_eq[wv] = static_cast<uint32_t>(__builtin_popcountll(m));
-      __syncthreads();
-      uint32_t before = 0, total = 0;
+    });
+    if (lane == 0) s_wave_eq[wv] = eq;
+    __syncthreads();
+    uint32_t run = 0u;  // keys == T before the current step
 #pragma unroll
-      for (int w2 = 0; w2 < NW; ++w2) {
-        const uint32_t c = s_wave_eq[w2];
-        before += w2 < wv ? c : 0u;
-        total += c;
+    for (int w2 = 0; w2 < NW; ++w2) run += w2 < wv ? s_wave_eq[w2] : 0u;
+    for (int v = v0; v < v1 && run < need; v += 64) {  // wave-uniform; a lane's four keys are adjacent
+      const u32x4_t kw = load_vec(v + lane);
+      uint32_t m4 = 0u;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) m4 |= (4 * (v + lane) + e < nv_i && v + lane < v1 && kw[e] == T) ? (1u << e) : 0u;
+      const uint32_t cnt = static_cast<uint32_t>(__builtin_popcount(m4));
+      uint32_t pos = run, tot = 0u;
+#pragma unroll
+      for (int bit = 0; bit < 3; ++bit) {
+        const uint64_t bm = __builtin_amdgcn_ballot_w64(((cnt >> bit) & 1u) != 0u);
+        pos += static_cast<uint32_t>(mbcnt64(bm)) << bit;
+        tot += static_cast<uint32_t>(__builtin_popcountll(bm)) << bit;
       }
-      if (eq) {
-        const uint32_t r = eq_run + before + static_cast<uint32_t>(mbcnt64(m));
-        if (r < need) sel[n_gt + r] = sort_word(key, static_cast<uint32_t>(j));
-      }
-      eq_run += total;
-      __syncthreads();
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if ((m4 >> e) & 1u) {
+          if (pos < need) sel[n_gt + pos] = sort_word(T, static_cast<uint32_t>(4 * (v + lane) + e));
+          ++pos;
+        }
+      run += tot;
     }
   }
   __syncthreads();
@@ -1196,6 +1238,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 512 ? 
 __host__ __device__ constexpr bool slot_cols_fit(int64_t S, int NT, int cols) {
   return (S + 15) / 16 <= static_cast<int64_t>(cols) * NT;
 }
+
+// The row strides and workspace pointers (and S) of a launch of B rows.
+void bind_workspace(MfmaIdxArgs& a, int64_t B, int64_t S, void* ws);
+// Enqueues the select of B rows whose order keys and slot maxima a score kernel has written.
+int launch_select(const MfmaIdxArgs& a, int64_t B, int64_t* out_idx, float* out_score, hipStream_t st, const char* who);
 
 // Launch set-up shared by the indexer and the fused CSA decode step: fills the kernel arguments
 // for B rows (T per key row), enqueues the score kernel and returns its status.
