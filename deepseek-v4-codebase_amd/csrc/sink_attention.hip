@@ -14,7 +14,7 @@
 //    gathers one tile of sources, dequantises the code rows on load to the same bf16 values
 //    PolarQuant.decode produces, attends them for all heads of the row and writes (max, sum, acc);
 //    the combine merges the tiles with the sink counted once.
-// 3. hca_compress_kernel — softmax over the M window positions and weighted sum
+// 3. hca_compress_rows_kernel, hca_compress_kernel — softmax over the M window positions and weighted sum
 //    (aether_kernels/sparse_attention.py:70-83; aether_2b/serving.py:495-497).
 #include <mutex>
 #include <unordered_set>
@@ -305,6 +305,142 @@ qattn_fn pick_qattn(int D) {
 // ------------------------------------------------------------------------------------------
 // 3. hca_compress
 // ------------------------------------------------------------------------------------------
+// Rows whose M entries fit in the registers of one team of lanes (a wave, or a workgroup of four):
+// bound by HBM (c and z read once).  A lane holds 16 bytes (VEC columns) of PER entries of z and of c, all
+// requested in one memory round; lane t of the team takes column chunk t % ncol and entries t / ncol,
+// t / ncol + MG, ..  (MG = team / ncol), so that a wave's loads cover whole rows.  The columns' maxima, then
+// the sums, are reduced over the lanes that share a chunk and, for a workgroup, over the waves through LDS.
+// Measured at 2048 x 128 x 128 bf16 (134 MB): 21.9 us = 6.1 TB/s with the inputs partly in the Infinity
+// Cache, 24.6 us = 5.5 TB/s on fresh ones, against 73 and 115 us with one lane per column reading z
+// twice, 2 bytes at a time; one row of 128 entries 3.8 us against 28 us.
+template <int DT>
+struct Vec16 {
+  static constexpr int N = 8;
+  __device__ static float get(const uint4& r, int e) {
+    const uint32_t w = e < 2 ? r.x : e < 4 ? r.y : e < 6 ? r.z : r.w;
+    const uint32_t b = (e & 1) ? w >> 16 : w & 0xffffu;
+    return DT == AEKV_BF16 ? bf16_to_f32(b) : f16_to_f32(b);
+  }
+};
+template <>
+struct Vec16<AEKV_F32> {
+  static constexpr int N = 4;
+  __device__ static float get(const uint4& r, int e) {
+    return __builtin_bit_cast(float, e == 0 ? r.x : e == 1 ? r.y : e == 2 ? r.z : r.w);
+  }
+};
+
+template <int DT, int PER, int WAVES>
+__global__ __launch_bounds__(kThreads) void hca_compress_rows_kernel(const uint4* __restrict__ c,
+                                                                     const uint4* __restrict__ z, int64_t B, int M,
+                                                                     int ncol, void* __restrict__ out) {
+  using V = Vec16<DT>;
+  constexpr int N = V::N;
+  __shared__ float s_max[WAVES == 1 ? 1 : 4][64 * N];
+  __shared__ float s_sum[WAVES == 1 ? 1 : 4][2][64 * N];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t b = WAVES == 1 ? static_cast<int64_t>(blockIdx.x) * 4 + wv : blockIdx.x;
+  if (WAVES == 1 && b >= B) return;  // wave-uniform, no barrier below for a team of one wave
+  const int t = WAVES == 1 ? lane : threadIdx.x;
+  const int col = t & (ncol - 1), m0 = t / ncol, MG = 64 * WAVES / ncol;
+  const int64_t base = b * M * ncol + col;
+  uint4 zr[PER], cr[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) zr[i] = z[base + static_cast<int64_t>(min(m0 + i * MG, M - 1)) * ncol];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) cr[i] = c[base + static_cast<int64_t>(min(m0 + i * MG, M - 1)) * ncol];
+  float mx[N], den[N], acc[N];
+#pragma unroll
+  for (int e = 0; e < N; ++e) {
+    mx[e] = kNegInf;
+#pragma unroll
+    for (int i = 0; i < PER; ++i)  // (an entry past M repeats the last one here)
+      mx[e] = fmaxf(mx[e], V::get(zr[i], e));
+  }
+  for (int hl = ncol; hl < 64; hl <<= 1) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) mx[e] = fmaxf(mx[e], xor_lane_rt(mx[e], hl));
+  }
+  if constexpr (WAVES > 1) {
+    if (lane < ncol) {
+#pragma unroll
+      for (int e = 0; e < N; ++e) s_max[wv][col * N + e] = mx[e];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < N; ++e)
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) mx[e] = fmaxf(mx[e], s_max[w][col * N + e]);
+  }
+#pragma unroll
+  for (int e = 0; e < N; ++e) {
+    den[e] = 0.0f;
+    acc[e] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const bool in = m0 + i * MG < M;
+      const float w = __expf(V::get(zr[i], e) - mx[e]);
+      den[e] += in ? w : 0.0f;
+      acc[e] = fmaf(in ? w : 0.0f, in ? V::get(cr[i], e) : 0.0f, acc[e]);
+    }
+  }
+  for (int hl = ncol; hl < 64; hl <<= 1) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+      den[e] += xor_lane_rt(den[e], hl);
+      acc[e] += xor_lane_rt(acc[e], hl);
+    }
+  }
+  const int64_t o = b * ncol * N;
+  if constexpr (WAVES > 1) {
+    if (lane < ncol) {
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        s_sum[wv][0][col * N + e] = den[e];
+        s_sum[wv][1][col * N + e] = acc[e];
+      }
+    }
+    __syncthreads();
+    for (int d = threadIdx.x; d < ncol * N; d += kThreads) {
+      float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) {
+        s0 += s_sum[w][0][d];
+        s1 += s_sum[w][1][d];
+      }
+      st<DT>(out, o + d, s1 / s0);
+    }
+  } else if (lane < ncol) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) st<DT>(out, o + col * N + e, acc[e] / den[e]);
+  }
+}
+
+// Launches the kernel above when the row's entries fit (at most 4 entries per lane of a wave, else at
+// most 16 per lane of a workgroup); false: nothing launched.
+template <int DT>
+bool launch_compress_rows(const void* c, const void* z, int64_t B, int64_t M, int64_t D, void* out, hipStream_t st) {
+  const int64_t ncol = D * static_cast<int64_t>(dtype_size(DT)) / 16;
+  if (ncol < 1 || ncol > 64 || !is_pow2(ncol) || D * static_cast<int64_t>(dtype_size(DT)) % 16 != 0 ||
+      !is_aligned(c, 16) || !is_aligned(z, 16) || B > 0x7fffffffLL)
+    return false;
+  const int64_t wave_groups = 64 / ncol, wg_groups = 256 / ncol;
+  const uint4* cv = static_cast<const uint4*>(c);
+  const uint4* zv = static_cast<const uint4*>(z);
+  auto go = [&](auto fn, int64_t grid) {
+    hipLaunchKernelGGL(fn, dim3(static_cast<uint32_t>(grid)), dim3(kThreads), 0, st, cv, zv, B, static_cast<int>(M),
+                       static_cast<int>(ncol), out);
+    return true;
+  };
+  if (M <= wave_groups) return go(hca_compress_rows_kernel<DT, 1, 1>, ceil_div(B, int64_t(4)));
+  if (M <= 2 * wave_groups) return go(hca_compress_rows_kernel<DT, 2, 1>, ceil_div(B, int64_t(4)));
+  if (M <= 4 * wave_groups) return go(hca_compress_rows_kernel<DT, 4, 1>, ceil_div(B, int64_t(4)));
+  if (M <= 4 * wg_groups) return go(hca_compress_rows_kernel<DT, 4, 4>, B);
+  if (M <= 8 * wg_groups) return go(hca_compress_rows_kernel<DT, 8, 4>, B);
+  if (M <= 16 * wg_groups) return go(hca_compress_rows_kernel<DT, 16, 4>, B);
+  return false;
+}
+
 template <int DT>
 __global__ __launch_bounds__(kThreads) void hca_compress_kernel(const void* __restrict__ c, const void* __restrict__ z,
                                                                 int64_t B, int64_t M, int64_t D, void* __restrict__ out) {
@@ -588,8 +724,12 @@ extern "C" int aekv_hca_compress(const void* c, const void* z, int32_t dtype, in
   if (B * D == 0) return AEKV_OK;
   if (M == 0) return fail(AEKV_ERR_SHAPE, "%s: empty compression window", who);
   if (!c || !z || !out) return fail(AEKV_ERR_VALUE, "%s: null pointer", who);
-  const dim3 grid(static_cast<uint32_t>(ceil_div(B * D, kThreads)));
   const hipStream_t st = as_stream(stream);
+  const bool rows = dtype == AEKV_F32   ? launch_compress_rows<AEKV_F32>(c, z, B, M, D, out, st)
+                    : dtype == AEKV_F16 ? launch_compress_rows<AEKV_F16>(c, z, B, M, D, out, st)
+                                        : launch_compress_rows<AEKV_BF16>(c, z, B, M, D, out, st);
+  if (rows) return check_launch(who);
+  const dim3 grid(static_cast<uint32_t>(ceil_div(B * D, kThreads)));
   if (dtype == AEKV_F32) hipLaunchKernelGGL(hca_compress_kernel<AEKV_F32>, grid, dim3(kThreads), 0, st, c, z, B, M, D, out);
   else if (dtype == AEKV_F16) hipLaunchKernelGGL(hca_compress_kernel<AEKV_F16>, grid, dim3(kThreads), 0, st, c, z, B, M, D, out);
   else hipLaunchKernelGGL(hca_compress_kernel<AEKV_BF16>, grid, dim3(kThreads), 0, st, c, z, B, M, D, out);
