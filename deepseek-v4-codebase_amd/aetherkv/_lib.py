@@ -35,7 +35,7 @@ SYMBOLS = (
     "aekv_set_flash_rows", "aekv_emit_block", "aekv_csa_prefill_indexer_topk_quant", "aekv_quant_prefill_workspace_size",
     "aekv_quant_prefill_attention", "aekv_rope_rmsnorm", "aekv_csa_indexer_topk_quant_noalloc",
     "aekv_csa_decode_workspace_size", "aekv_csa_decode_quant", "aekv_sparse_sink_attention_ws",
-    "aekv_tiled_prefill_attention_ws", "aekv_sink_attention_workspace_size",
+    "aekv_tiled_prefill_attention_ws", "aekv_sink_attention_workspace_size", "aekv_prefill_counts",
 )
 
 # size of the static device scratch behind aekv_csa_indexer_topk_quant_noalloc (AEKV_STATIC_SCRATCH_BYTES)
@@ -101,6 +101,7 @@ def lib() -> ctypes.CDLL:
             [P, P, P, I32_, P, I64_, I32_, I64_, I64_, I64_, I64_, I64_, I64_, F, P, SZ, P, P], ctypes.c_int),
         "aekv_tiled_prefill_attention_ws": (
             [P, P, P, I64_, I32_, I64_, I64_, I64_, I64_, I64_, F, I32_, P, SZ, P, P], ctypes.c_int),
+        "aekv_prefill_counts": ([I64_] * 8 + [P, P, P, P, P], ctypes.c_int),
         "aekv_sink_attention_workspace_size": ([I32_, I64_, I64_, I64_, I64_, I64_, I64_], SZ),
     }
     for name, (argtypes, restype) in sig.items():

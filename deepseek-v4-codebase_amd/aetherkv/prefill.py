@@ -11,7 +11,7 @@ bf16 compressed blocks.  Here the blocks stay TurboQuant codes: one indexer laun
 target of the chunk (each against its own visible prefix), and one attention launch covers every
 (target, head) row, gathering and dequantising the code rows on load; each target reads its own
 slice of one window buffer.  The positional bookkeeping (which blocks and window entries a target
-sees) follows the reference exactly and is computed on the host (:316-320, :521-534).
+sees) follows the reference exactly (:316-320, :521-534) and is computed on the device.
 
 Not covered here: the query-side projections and the inverse RoPE / output projection around the
 attention call (:326-337, :540-550) — callers keep those.
@@ -36,19 +36,25 @@ def prefill_sources(n_targets: int, start: int, n_blocks: int, *, compression: i
     as (start, length) relative to a window buffer whose entry i holds position window_base + i and
     which holds window_len entries.  Raises ValueError if the buffer does not cover a slice.
     """
-    if n_targets < 0 or start < 0 or n_blocks < 0:
-        raise ValueError("n_targets, start and n_blocks must be non-negative")
-    if compression < 1 or sliding_window < 1:
-        raise ValueError("compression and sliding_window must be positive")
+    _check_chunk(n_targets, start, n_blocks, compression, sliding_window, window_base, window_len)
     p = torch.arange(start, start + n_targets, dtype=torch.int64)
     vis = torch.clamp(p // compression, max=n_blocks)
     w_first = torch.clamp(p - sliding_window + 1, min=0)
     ws = w_first - window_base
     wl = p - w_first + 1
-    if n_targets and (int(ws.min()) < 0 or int((ws + wl).max()) > window_len):
+    return vis.to(torch.int32), ws.to(torch.int32), wl.to(torch.int32)
+
+
+def _check_chunk(n_targets: int, start: int, n_blocks: int, compression: int, sliding_window: int, window_base: int,
+                 window_len: int) -> None:
+    if n_targets < 0 or start < 0 or n_blocks < 0:
+        raise ValueError("n_targets, start and n_blocks must be non-negative")
+    if compression < 1 or sliding_window < 1:
+        raise ValueError("compression and sliding_window must be positive")
+    # the first target's slice starts earliest, the last one's ends last
+    if n_targets and (max(0, start - sliding_window + 1) < window_base or start + n_targets - window_base > window_len):
         raise ValueError(f"window buffer of {window_len} entries from position {window_base} does not cover the "
                          f"sliding windows of positions {start} .. {start + n_targets - 1}")
-    return vis.to(torch.int32), ws.to(torch.int32), wl.to(torch.int32)
 
 
 def prefill_workspace(B: int, T: int, H: int, n_comp: int, Wt: int, device) -> torch.Tensor:
@@ -178,13 +184,23 @@ def quant_prefill_attention(q: torch.Tensor, codes: torch.Tensor, scale: torch.T
     return out
 
 
-def _window_rows(window: torch.Tensor, T: int, start: int, n_blocks: int, compression: int, sliding_window: int,
-                 window_base: Optional[int]):
-    Wt = window.size(1)
+def _device_sources(q: torch.Tensor, window: torch.Tensor, start: int, n_blocks: int, compression: int,
+                    sliding_window: int, window_base: Optional[int], k: int) -> torch.Tensor:
+    """prefill_sources of every row of q [B, T, ...] as int32 [4, B, T] on its device: visible blocks,
+    those capped at k, window start and length (one launch; arrays made on the host would be copied
+    synchronously)."""
+    (B, T), Wt = q.shape[:2], window.size(1)
+    start, n_blocks, compression, sliding_window = int(start), int(n_blocks), int(compression), int(sliding_window)
     base = start + T - Wt if window_base is None else int(window_base)
-    vis, ws, wl = prefill_sources(T, start, n_blocks, compression=compression, sliding_window=sliding_window,
-                                  window_base=base, window_len=Wt)
-    return vis, ws, wl
+    _check_chunk(T, start, n_blocks, compression, sliding_window, base, Wt)
+    _lib.require_device("q", q)
+    rows = torch.empty((4, B, T), dtype=torch.int32, device=q.device)
+    at, step = rows.data_ptr(), 4 * B * T
+    with _lib.on_device(q.device):
+        rc = _lib.lib().aekv_prefill_counts(B, T, start, n_blocks, compression, sliding_window, base, max(k, 0), at,
+                                            at + step, at + 2 * step, at + 3 * step, _lib.raw_stream(q.device))
+    _lib.check(rc, "aekv_prefill_counts")
+    return rows
 
 
 def hca_prefill(q: torch.Tensor, kv_codes: torch.Tensor, kv_scale: torch.Tensor, window: torch.Tensor,
@@ -198,12 +214,10 @@ def hca_prefill(q: torch.Tensor, kv_codes: torch.Tensor, kv_scale: torch.Tensor,
     ends at the chunk's last target).  Returns the per-target attention [B, T, H, 128] bf16, before
     the reference's inverse RoPE and output projection.
     """
-    B, T = q.shape[:2]
     nb = kv_codes.size(1) if n_blocks is None else int(n_blocks)
-    vis, ws, wl = _window_rows(window, T, start, nb, compression, sliding_window, window_base)
-    dev = q.device
+    vis, _, ws, wl = _device_sources(q, window, start, nb, compression, sliding_window, window_base, 0)
     return quant_prefill_attention(q, kv_codes, kv_scale, None, window, sink, softmax_scale, quant=kv_quant,
-                                   visible=vis.to(dev), win_start=ws.to(dev), win_len=wl.to(dev))
+                                   visible=vis, win_start=ws, win_len=wl)
 
 
 def csa_prefill(q: torch.Tensor, index_q: torch.Tensor, index_weight: torch.Tensor, index_codes: torch.Tensor,
@@ -223,17 +237,15 @@ def csa_prefill(q: torch.Tensor, index_q: torch.Tensor, index_weight: torch.Tens
     B, T = q.shape[:2]
     nb = kv_codes.size(1) if n_blocks is None else int(n_blocks)
     k_cfg = min(int(top_k), nb) if nb > 0 else 0  # modeling.py:511
-    vis, ws, wl = _window_rows(window, T, start, nb, compression, sliding_window, window_base)
-    dev = q.device
+    # (n_sel: k_eff = min(K, g), modeling.py:527)
+    vis, n_sel, ws, wl = _device_sources(q, window, start, nb, compression, sliding_window, window_base, k_cfg)
     if k_cfg == 0:
         idx = None
-        sel = torch.zeros((B, T, 0), dtype=torch.int64, device=dev)
-        n_sel = torch.zeros_like(vis)
+        sel = torch.zeros((B, T, 0), dtype=torch.int64, device=q.device)
     else:
         idx = csa_prefill_indexer_topk_quant(index_q, index_weight, index_codes, index_scale, k_cfg,
-                                             quant=index_quant, valid=vis.to(dev), mode=mode)
+                                             quant=index_quant, valid=vis, mode=mode)
         sel = idx
-        n_sel = torch.clamp(vis, max=k_cfg)  # k_eff = min(K, g), modeling.py:527
     out = quant_prefill_attention(q, kv_codes, kv_scale, sel, window, sink, softmax_scale, quant=kv_quant,
-                                  visible=n_sel.to(dev), win_start=ws.to(dev), win_len=wl.to(dev))
+                                  visible=n_sel, win_start=ws, win_len=wl)
     return out, idx

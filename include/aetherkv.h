@@ -229,6 +229,15 @@ int aekv_quant_prefill_attention(const void* q, const void* codes, const float* 
                                  int32_t bits, float softmax_scale, void* ws, size_t ws_bytes, void* out,
                                  void* stream);
 
+/* Per-target source counts of a prefill chunk, computed on the device (modeling.py:316-319, :521-534):
+ * for target t of each of B sequences, at position p = start + t, visible[b,t] = min(n_blocks,
+ * p / compression), selected[b,t] = min(visible, k) (nullable), and its window slice [max(0, p -
+ * sliding_window + 1), p] as win_start[b,t] (relative to position window_base) and win_len[b,t].  All
+ * [B,T] int32.  The caller checks that the window buffer covers the slices. */
+int aekv_prefill_counts(int64_t B, int64_t T, int64_t start, int64_t n_blocks, int64_t compression,
+                        int64_t sliding_window, int64_t window_base, int64_t k, int32_t* visible,
+                        int32_t* selected, int32_t* win_start, int32_t* win_len, void* stream);
+
 /* One CSA decode step over TurboQuant-coded caches (aether_2b/serving.py:597-625: score every
  * visible block of the index cache, topk, gather the selected KV blocks, concat the window, attend
  * with the per-head sink): aekv_csa_indexer_topk_quant's selection (out_idx [B, k] int64, -1 padded,
