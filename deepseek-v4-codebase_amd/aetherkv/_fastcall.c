@@ -1,4 +1,4 @@
-/* Direct CPython calls of the libaetherkv C ABI entry points that callers make once per token.
+/* Direct CPython calls of the libaetherkv C ABI entry points that callers make once per token or chunk.
  *
  * The reference's model calls tiled_prefill_attention once per target token (aether_2b/modeling.py:
  * 322,534) and its engine calls sparse_sink_attention / the decode step once per layer and token, so
@@ -138,7 +138,136 @@ static PyObject* f_csa_decode_quant(PyObject* self, PyObject* const* args, Py_ss
                                       (float*)os, out, st));
 }
 
+/* aekv_tq_encode(x, x_dtype, n_vec, d, bits, diag, codes, scale, stream) */
+static PyObject* f_tq_encode(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+  (void)self;
+  if (want_args(nargs, 9, "aekv_tq_encode")) return NULL;
+  void* x = ptr_arg(A(0));
+  const int32_t dt = i32_arg(A(1));
+  const int64_t n = i64_arg(A(2));
+  const int32_t d = i32_arg(A(3)), bits = i32_arg(A(4));
+  void* diag = ptr_arg(A(5));
+  void* codes = ptr_arg(A(6));
+  void* scale = ptr_arg(A(7));
+  void* st = ptr_arg(A(8));
+  RETURN_STATUS(aekv_tq_encode(x, dt, n, d, bits, (const float*)diag, codes, (float*)scale, st));
+}
+
+/* aekv_tq_decode(codes, scale, n_vec, d, bits, diag, out, out_dtype, stream) */
+static PyObject* f_tq_decode(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+  (void)self;
+  if (want_args(nargs, 9, "aekv_tq_decode")) return NULL;
+  void* codes = ptr_arg(A(0));
+  void* scale = ptr_arg(A(1));
+  const int64_t n = i64_arg(A(2));
+  const int32_t d = i32_arg(A(3)), bits = i32_arg(A(4));
+  void* diag = ptr_arg(A(5));
+  void* out = ptr_arg(A(6));
+  const int32_t odt = i32_arg(A(7));
+  void* st = ptr_arg(A(8));
+  RETURN_STATUS(aekv_tq_decode(codes, (const float*)scale, n, d, bits, (const float*)diag, out, odt, st));
+}
+
+/* aekv_hca_compress(c, z, dtype, B, M, D, out, stream) */
+static PyObject* f_hca_compress(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+  (void)self;
+  if (want_args(nargs, 8, "aekv_hca_compress")) return NULL;
+  void* c = ptr_arg(A(0));
+  void* z = ptr_arg(A(1));
+  const int32_t dt = i32_arg(A(2));
+  const int64_t B = i64_arg(A(3)), M = i64_arg(A(4)), D = i64_arg(A(5));
+  void* out = ptr_arg(A(6));
+  void* st = ptr_arg(A(7));
+  RETURN_STATUS(aekv_hca_compress(c, z, dt, B, M, D, out, st));
+}
+
+/* aekv_csa_indexer_topk(index_q, index_kv, index_weight, valid, B, S, IH, IC, k, mode, ws, ws_bytes, out_idx,
+ * out_score, stream) */
+static PyObject* f_csa_indexer_topk(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+  (void)self;
+  if (want_args(nargs, 15, "aekv_csa_indexer_topk")) return NULL;
+  void* q = ptr_arg(A(0));
+  void* kv = ptr_arg(A(1));
+  void* w = ptr_arg(A(2));
+  void* valid = ptr_arg(A(3));
+  const int64_t B = i64_arg(A(4)), S = i64_arg(A(5));
+  const int32_t IH = i32_arg(A(6)), IC = i32_arg(A(7)), k = i32_arg(A(8)), mode = i32_arg(A(9));
+  void* ws = ptr_arg(A(10));
+  const size_t wsb = (size_t)i64_arg(A(11));
+  void* oi = ptr_arg(A(12));
+  void* os = ptr_arg(A(13));
+  void* st = ptr_arg(A(14));
+  RETURN_STATUS(aekv_csa_indexer_topk((const float*)q, (const float*)kv, (const float*)w, (const int32_t*)valid, B, S, IH,
+                                      IC, k, mode, ws, wsb, (int64_t*)oi, (float*)os, st));
+}
+
+/* aekv_csa_prefill_indexer_topk_quant(index_q, index_weight, key_codes, key_scale, diag, valid, B, T, S, IH, IC, bits, k,
+ * mode, ws, ws_bytes, out_idx, out_score, stream) */
+static PyObject* f_csa_prefill_indexer(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+  (void)self;
+  if (want_args(nargs, 19, "aekv_csa_prefill_indexer_topk_quant")) return NULL;
+  void* q = ptr_arg(A(0));
+  void* w = ptr_arg(A(1));
+  void* kc = ptr_arg(A(2));
+  void* ks = ptr_arg(A(3));
+  void* diag = ptr_arg(A(4));
+  void* valid = ptr_arg(A(5));
+  const int64_t B = i64_arg(A(6)), T = i64_arg(A(7)), S = i64_arg(A(8));
+  const int32_t IH = i32_arg(A(9)), IC = i32_arg(A(10)), bits = i32_arg(A(11)), k = i32_arg(A(12)), mode = i32_arg(A(13));
+  void* ws = ptr_arg(A(14));
+  const size_t wsb = (size_t)i64_arg(A(15));
+  void* oi = ptr_arg(A(16));
+  void* os = ptr_arg(A(17));
+  void* st = ptr_arg(A(18));
+  RETURN_STATUS(aekv_csa_prefill_indexer_topk_quant((const float*)q, (const float*)w, kc, (const float*)ks,
+                                                    (const float*)diag, (const int32_t*)valid, B, T, S, IH, IC, bits, k,
+                                                    mode, ws, wsb, (int64_t*)oi, (float*)os, st));
+}
+
+/* aekv_quant_prefill_attention(q, codes, scale, sel, visible, window, win_start, win_len, sink, diag, B, T, H, D, S,
+ * n_sel, Wt, bits, scale, ws, ws_bytes, out, stream) */
+static PyObject* f_quant_prefill_attention(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+  (void)self;
+  if (want_args(nargs, 23, "aekv_quant_prefill_attention")) return NULL;
+  void* p[10];
+  for (int i = 0; i < 10; ++i) p[i] = ptr_arg(A(i));
+  const int64_t B = i64_arg(A(10)), T = i64_arg(A(11)), H = i64_arg(A(12)), D = i64_arg(A(13)), S = i64_arg(A(14));
+  const int64_t ns = i64_arg(A(15)), Wt = i64_arg(A(16));
+  const int32_t bits = i32_arg(A(17));
+  const float sm = f32_arg(A(18));
+  void* ws = ptr_arg(A(19));
+  const size_t wsb = (size_t)i64_arg(A(20));
+  void* out = ptr_arg(A(21));
+  void* st = ptr_arg(A(22));
+  RETURN_STATUS(aekv_quant_prefill_attention(p[0], p[1], (const float*)p[2], (const int64_t*)p[3], (const int32_t*)p[4],
+                                             p[5], (const int32_t*)p[6], (const int32_t*)p[7], (const float*)p[8],
+                                             (const float*)p[9], B, T, H, D, S, ns, Wt, bits, sm, ws, wsb, out, st));
+}
+
+/* aekv_prefill_counts(B, T, start, n_blocks, compression, sliding_window, window_base, k, visible, selected, win_start,
+ * win_len, stream) */
+static PyObject* f_prefill_counts(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+  (void)self;
+  if (want_args(nargs, 13, "aekv_prefill_counts")) return NULL;
+  int64_t n[8];
+  for (int i = 0; i < 8; ++i) n[i] = i64_arg(A(i));
+  void* vis = ptr_arg(A(8));
+  void* sel = ptr_arg(A(9));
+  void* ws = ptr_arg(A(10));
+  void* wl = ptr_arg(A(11));
+  void* st = ptr_arg(A(12));
+  RETURN_STATUS(aekv_prefill_counts(n[0], n[1], n[2], n[3], n[4], n[5], n[6], n[7], (int32_t*)vis, (int32_t*)sel,
+                                    (int32_t*)ws, (int32_t*)wl, st));
+}
+
 static PyMethodDef methods[] = {
+    {"aekv_tq_encode", (PyCFunction)(void (*)(void))f_tq_encode, METH_FASTCALL, NULL},
+    {"aekv_tq_decode", (PyCFunction)(void (*)(void))f_tq_decode, METH_FASTCALL, NULL},
+    {"aekv_hca_compress", (PyCFunction)(void (*)(void))f_hca_compress, METH_FASTCALL, NULL},
+    {"aekv_csa_indexer_topk", (PyCFunction)(void (*)(void))f_csa_indexer_topk, METH_FASTCALL, NULL},
+    {"aekv_csa_prefill_indexer_topk_quant", (PyCFunction)(void (*)(void))f_csa_prefill_indexer, METH_FASTCALL, NULL},
+    {"aekv_quant_prefill_attention", (PyCFunction)(void (*)(void))f_quant_prefill_attention, METH_FASTCALL, NULL},
+    {"aekv_prefill_counts", (PyCFunction)(void (*)(void))f_prefill_counts, METH_FASTCALL, NULL},
     {"aekv_sparse_sink_attention_ws", (PyCFunction)(void (*)(void))f_sparse_sink_attention_ws, METH_FASTCALL, NULL},
     {"aekv_tiled_prefill_attention_ws", (PyCFunction)(void (*)(void))f_tiled_prefill_attention_ws, METH_FASTCALL, NULL},
     {"aekv_quant_sink_attention", (PyCFunction)(void (*)(void))f_quant_sink_attention, METH_FASTCALL, NULL},

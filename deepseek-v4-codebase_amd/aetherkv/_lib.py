@@ -11,6 +11,7 @@ There is no fallback: if the library is missing every entry point raises.
 from __future__ import annotations
 
 import ctypes
+import functools
 from pathlib import Path
 from typing import Optional
 
@@ -195,6 +196,23 @@ def workspace(nbytes: int, device: torch.device, stream: int) -> Optional[torch.
     buf = torch.empty(max(nbytes, 2 * buf.numel() if buf is not None else 0), dtype=torch.uint8, device=device)
     _ws_cache[key] = buf
     return buf
+
+
+# Workspace sizes that depend on the call's sizes alone, memoised: the calls that use them run once per
+# layer and token.  (The prefill attention's also depends on the device and on aekv_set_flash_rows.)
+@functools.lru_cache(maxsize=1024)
+def indexer_ws_bytes(B: int, S: int, k: int) -> int:
+    return lib().aekv_csa_indexer_workspace_size(B, S, k)
+
+
+@functools.lru_cache(maxsize=1024)
+def attention_ws_bytes(B: int, H: int, D: int, n_comp: int, W: int) -> int:
+    return lib().aekv_quant_attention_workspace_size(B, H, D, n_comp, W)
+
+
+@functools.lru_cache(maxsize=1024)
+def decode_ws_bytes(B: int, S: int, k: int, H: int, D: int, W: int) -> int:
+    return lib().aekv_csa_decode_workspace_size(B, S, k, H, D, W)
 
 
 def require_device(name: str, *tensors: Optional[torch.Tensor]) -> None:

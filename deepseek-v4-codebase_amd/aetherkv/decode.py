@@ -100,12 +100,11 @@ def _prefix_rows(codes: torch.Tensor, scale: torch.Tensor) -> Optional[int]:
 
 
 def indexer_workspace(B: int, S: int, k: int, device) -> torch.Tensor:
-    return torch.empty(_lib.lib().aekv_csa_indexer_workspace_size(B, S, k), dtype=torch.uint8, device=device)
+    return torch.empty(_lib.indexer_ws_bytes(B, S, k), dtype=torch.uint8, device=device)
 
 
 def attention_workspace(B: int, H: int, D: int, n_comp: int, W: int, device) -> torch.Tensor:
-    return torch.empty(_lib.lib().aekv_quant_attention_workspace_size(B, H, D, n_comp, W), dtype=torch.uint8,
-                       device=device)
+    return torch.empty(_lib.attention_ws_bytes(B, H, D, n_comp, W), dtype=torch.uint8, device=device)
 
 
 def csa_indexer_topk_quant(index_q: torch.Tensor, index_weight: torch.Tensor, key_codes: torch.Tensor,
@@ -216,7 +215,7 @@ def quant_sink_attention(q: torch.Tensor, codes: torch.Tensor, scale: torch.Tens
 
 def decode_workspace(B: int, S: int, k: int, H: int, D: int, W: int, device) -> torch.Tensor:
     """Workspace of csa_decode_step (the indexer's and the attention's)."""
-    return torch.empty(_lib.lib().aekv_csa_decode_workspace_size(B, S, k, H, D, W), dtype=torch.uint8, device=device)
+    return torch.empty(_lib.decode_ws_bytes(B, S, k, H, D, W), dtype=torch.uint8, device=device)
 
 
 def csa_decode_step(q: torch.Tensor, index_q: torch.Tensor, index_weight: torch.Tensor, index_codes: torch.Tensor,
@@ -273,7 +272,6 @@ def csa_decode_step(q: torch.Tensor, index_q: torch.Tensor, index_weight: torch.
     dev = q.device
     idiag = index_quant._diag(IC, dev)
     kdiag = kv_quant._diag(D, dev)
-    L = _lib.lib()
     if out_idx is None:
         out_idx = torch.empty((B, k), dtype=torch.int64, device=dev)
     else:

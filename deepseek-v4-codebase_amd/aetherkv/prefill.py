@@ -23,7 +23,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib
-from .decode import _scale_2d
+from .decode import _f32, _iptr, _scale_2d, _sink_f32
 from .turbo_quant import PolarQuant
 
 
@@ -65,7 +65,8 @@ def prefill_workspace(B: int, T: int, H: int, n_comp: int, Wt: int, device) -> t
 def _rows_i32(x: Optional[torch.Tensor], B: int, T: int, name: str, device) -> Optional[torch.Tensor]:
     if x is None:
         return None
-    x = x.to(device=device, dtype=torch.int32)
+    if x.dtype != torch.int32 or x.device != device:
+        x = x.to(device=device, dtype=torch.int32)
     if x.dim() == 1:
         x = x.expand(B, T)
     if tuple(x.shape) != (B, T):
@@ -99,24 +100,24 @@ def csa_prefill_indexer_topk_quant(index_q: torch.Tensor, index_weight: torch.Te
         raise RuntimeError(f"key_codes shape {tuple(key_codes.shape)} does not match index_q {tuple(index_q.shape)}")
     if tuple(index_weight.shape) != (B, T, IH):
         raise RuntimeError(f"index_weight must be [B, T, IH] = [{B}, {T}, {IH}], got {tuple(index_weight.shape)}")
-    q = index_q.to(torch.float32).contiguous()
-    w = index_weight.to(torch.float32).contiguous()
+    q = _f32(index_q)
+    w = _f32(index_weight)
     codes = key_codes.contiguous()
     sc = _scale_2d(key_scale, B, S)
-    v = _rows_i32(valid, B, T, "valid", index_q.device)
-    diag = quant._diag(IC, index_q.device)
-    L = _lib.lib()
+    dev = index_q.device
+    v = _rows_i32(valid, B, T, "valid", dev)
+    diag = quant._diag(IC, dev)
     if out is None:
-        out = torch.empty((B, T, k), dtype=torch.int64, device=index_q.device)
-    scores = torch.empty((B, T, k), dtype=torch.float32, device=index_q.device) if return_scores else None
+        out = torch.empty((B, T, k), dtype=torch.int64, device=dev)
+    scores = torch.empty((B, T, k), dtype=torch.float32, device=dev) if return_scores else None
     if workspace is None:
-        workspace = torch.empty(L.aekv_csa_indexer_workspace_size(B * T, S, k), dtype=torch.uint8,
-                                device=index_q.device)
-    with torch.cuda.device(index_q.device):
-        _lib.check(L.aekv_csa_prefill_indexer_topk_quant(
-            _lib.ptr(q), _lib.ptr(w), _lib.ptr(codes), _lib.ptr(sc), _lib.ptr(diag), _lib.ptr(v), B, T, S, IH, IC,
-            bits, int(k), _lib.INDEX_MODES[mode], _lib.ptr(workspace), workspace.numel(), _lib.ptr(out),
-            _lib.ptr(scores), _lib.stream_of(index_q)), "aekv_csa_prefill_indexer_topk_quant")
+        workspace = torch.empty(_lib.indexer_ws_bytes(B * T, S, k), dtype=torch.uint8, device=dev)
+    with _lib.on_device(dev):
+        rc = _lib.hot("aekv_csa_prefill_indexer_topk_quant")(
+            q.data_ptr(), w.data_ptr(), codes.data_ptr(), sc.data_ptr(), diag.data_ptr(), _iptr(v), B, T, S, IH, IC, bits,
+            int(k), _lib.INDEX_MODES[mode], workspace.data_ptr(), workspace.numel(), out.data_ptr(), _iptr(scores),
+            _lib.raw_stream(dev))
+    _lib.check(rc, "aekv_csa_prefill_indexer_topk_quant")
     return (out, scores) if return_scores else out
 
 
@@ -162,11 +163,7 @@ def quant_prefill_attention(q: torch.Tensor, codes: torch.Tensor, scale: torch.T
         Wt = win.size(1)
     else:
         win, Wt = None, 0
-    sk = sink.to(torch.float32).reshape(-1).contiguous()
-    if sk.numel() == 1:
-        sk = sk.expand(H).contiguous()
-    if sk.numel() != H:
-        raise RuntimeError("sink must be a scalar or a [num_heads] tensor")
+    sk = _sink_f32(sink, H)
     vis = _rows_i32(visible, B, T, "visible", q.device)
     ws_ = _rows_i32(win_start, B, T, "win_start", q.device)
     wl = _rows_i32(win_len, B, T, "win_len", q.device)
@@ -176,11 +173,13 @@ def quant_prefill_attention(q: torch.Tensor, codes: torch.Tensor, scale: torch.T
         workspace = prefill_workspace(B, T, H, n_comp, Wt, q.device)
     if out is None:
         out = torch.empty((B, T, H, D), dtype=torch.bfloat16, device=q.device)
-    with torch.cuda.device(q.device):
-        _lib.check(_lib.lib().aekv_quant_prefill_attention(
-            _lib.ptr(qc), _lib.ptr(cc), _lib.ptr(sc), _lib.ptr(s64), _lib.ptr(vis), _lib.ptr(win), _lib.ptr(ws_),
-            _lib.ptr(wl), _lib.ptr(sk), _lib.ptr(diag), B, T, H, D, S, K, Wt, bits, float(softmax_scale),
-            _lib.ptr(workspace), workspace.numel(), _lib.ptr(out), _lib.stream_of(q)), "aekv_quant_prefill_attention")
+    dev = q.device
+    with _lib.on_device(dev):
+        rc = _lib.hot("aekv_quant_prefill_attention")(
+            qc.data_ptr(), cc.data_ptr(), sc.data_ptr(), _iptr(s64), _iptr(vis), _iptr(win), _iptr(ws_), _iptr(wl),
+            sk.data_ptr(), diag.data_ptr(), B, T, H, D, S, K, Wt, bits, float(softmax_scale), workspace.data_ptr(),
+            workspace.numel(), out.data_ptr(), _lib.raw_stream(dev))
+    _lib.check(rc, "aekv_quant_prefill_attention")
     return out
 
 
@@ -197,8 +196,8 @@ def _device_sources(q: torch.Tensor, window: torch.Tensor, start: int, n_blocks:
     rows = torch.empty((4, B, T), dtype=torch.int32, device=q.device)
     at, step = rows.data_ptr(), 4 * B * T
     with _lib.on_device(q.device):
-        rc = _lib.lib().aekv_prefill_counts(B, T, start, n_blocks, compression, sliding_window, base, max(k, 0), at,
-                                            at + step, at + 2 * step, at + 3 * step, _lib.raw_stream(q.device))
+        rc = _lib.hot("aekv_prefill_counts")(B, T, start, n_blocks, compression, sliding_window, base, max(k, 0), at,
+                                             at + step, at + 2 * step, at + 3 * step, _lib.raw_stream(q.device))
     _lib.check(rc, "aekv_prefill_counts")
     return rows
 

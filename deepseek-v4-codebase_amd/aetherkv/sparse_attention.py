@@ -179,14 +179,14 @@ def _ext_csa_indexer_topk(index_q, index_kv, index_weight, k, mode="relu_w"):
         raise RuntimeError("index_q, index_kv and index_weight shapes do not match")
     if mode not in _lib.INDEX_MODES:
         raise ValueError(f"mode must be one of {sorted(_lib.INDEX_MODES)}, got {mode!r}")
-    L = _lib.lib()
-    out = torch.empty((B, k), dtype=torch.int64, device=index_q.device)
-    ws = torch.empty(L.aekv_csa_indexer_workspace_size(B, S, k), dtype=torch.uint8, device=index_q.device)
-    with torch.cuda.device(index_q.device):
-        _lib.check(L.aekv_csa_indexer_topk(
-            _lib.ptr(index_q), _lib.ptr(index_kv), _lib.ptr(index_weight), None, B, S, IH, IC, int(k),
-            _lib.INDEX_MODES[mode], _lib.ptr(ws), ws.numel(), _lib.ptr(out), None, _lib.stream_of(index_q)),
-            "aekv_csa_indexer_topk")
+    dev = index_q.device
+    out = torch.empty((B, k), dtype=torch.int64, device=dev)
+    ws = torch.empty(_lib.indexer_ws_bytes(B, S, k), dtype=torch.uint8, device=dev)
+    with _lib.on_device(dev):
+        rc = _lib.hot("aekv_csa_indexer_topk")(
+            index_q.data_ptr(), index_kv.data_ptr(), index_weight.data_ptr(), None, B, S, IH, IC, int(k),
+            _lib.INDEX_MODES[mode], ws.data_ptr(), ws.numel(), out.data_ptr(), None, _lib.raw_stream(dev))
+    _lib.check(rc, "aekv_csa_indexer_topk")
     return out
 
 
@@ -203,10 +203,12 @@ def _ext_hca_compress(buffer_c, buffer_z):
     if buffer_z.dtype != buffer_c.dtype:
         raise RuntimeError("buffer_c and buffer_z must share one floating dtype")
     B, M, D = buffer_c.shape
-    out = torch.empty((B, D), dtype=buffer_c.dtype, device=buffer_c.device)
-    with torch.cuda.device(buffer_c.device):
-        _lib.check(_lib.lib().aekv_hca_compress(_lib.ptr(buffer_c), _lib.ptr(buffer_z), _lib.dtype_code(buffer_c), B, M,
-                                                D, _lib.ptr(out), _lib.stream_of(buffer_c)), "aekv_hca_compress")
+    dev = buffer_c.device
+    out = torch.empty((B, D), dtype=buffer_c.dtype, device=dev)
+    with _lib.on_device(dev):
+        rc = _lib.hot("aekv_hca_compress")(buffer_c.data_ptr(), buffer_z.data_ptr(), _lib.dtype_code(buffer_c), B, M, D,
+                                           out.data_ptr(), _lib.raw_stream(dev))
+    _lib.check(rc, "aekv_hca_compress")
     return out
 
 

@@ -52,16 +52,17 @@ class PolarQuant:
             raise ValueError(f"bits must be 4 or 8, got {bits}")
         self.bits = bits
         self._seed = seed
-        self._diag_cache: Dict[Tuple[int, str], torch.Tensor] = {}
+        self._diag_cache: Dict[Tuple[int, torch.device], torch.Tensor] = {}
 
     def _diag(self, d: int, device: torch.device) -> torch.Tensor:
         """Fixed +-1 diagonal for dimension d: MT19937(seed*10007+d) draws, r > 0.5 -> +1."""
-        key = (d, str(device))
-        if key not in self._diag_cache:
+        key = (d, device)
+        diag = self._diag_cache.get(key)
+        if diag is None:
             host = torch.empty(d, dtype=torch.float32)
             _lib.check(_lib.lib().aekv_tq_diag(self._seed, d, _lib.ptr(host)), "aekv_tq_diag")
-            self._diag_cache[key] = host.to(device)
-        return self._diag_cache[key]
+            diag = self._diag_cache[key] = host.to(device)
+        return diag
 
     def encode(self, x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
         """x [..., D] -> (int8 [..., D] | uint8 [..., D//2], fp32 scale [..., 1])."""
@@ -70,20 +71,19 @@ class PolarQuant:
         _lib.require_device("x", x)
         if x.dtype not in (torch.float32, torch.float16, torch.bfloat16):
             x = x.to(torch.float32)
-        diag = self._diag(d, x.device)
-        epl = min(d, 8)
-        src = _lib.aligned(x, min(16, epl * x.element_size()))
-        lead = tuple(x.shape[:-1])
+        dev = x.device
+        diag = self._diag(d, dev)
+        src = _lib.aligned(x, min(16, min(d, 8) * x.element_size()))
+        lead = x.shape[:-1]
         if self.bits == 8:
-            data = torch.empty(lead + (d,), dtype=torch.int8, device=x.device)
+            data = torch.empty(lead + (d,), dtype=torch.int8, device=dev)
         else:
-            data = torch.empty(lead + (d // 2,), dtype=torch.uint8, device=x.device)
-        scale = torch.empty(lead + (1,), dtype=torch.float32, device=x.device)
-        n = x.numel() // d
-        with torch.cuda.device(x.device):
-            _lib.check(_lib.lib().aekv_tq_encode(_lib.ptr(src), _lib.dtype_code(src), n, d, self.bits, _lib.ptr(diag),
-                                                 _lib.ptr(data), _lib.ptr(scale), _lib.stream_of(x)),
-                       "aekv_tq_encode")
+            data = torch.empty(lead + (d // 2,), dtype=torch.uint8, device=dev)
+        scale = torch.empty(lead + (1,), dtype=torch.float32, device=dev)
+        with _lib.on_device(dev):
+            rc = _lib.hot("aekv_tq_encode")(src.data_ptr(), _lib.TORCH_TO_AEKV[src.dtype], x.numel() // d, d, self.bits,
+                                            diag.data_ptr(), data.data_ptr(), scale.data_ptr(), _lib.raw_stream(dev))
+        _lib.check(rc, "aekv_tq_encode")
         return data, scale
 
     def decode(self, data: torch.Tensor, scale: torch.Tensor,
@@ -95,20 +95,20 @@ class PolarQuant:
             raise RuntimeError(f"{self.bits}-bit PolarQuant codes must be {want}, got {data.dtype}")
         d = data.shape[-1] * (1 if self.bits == 8 else 2)
         _check_pow2(d)
-        lead = tuple(data.shape[:-1])
+        lead = data.shape[:-1]
         n = data.numel() // max(data.shape[-1], 1)
-        scale_f32 = scale.to(torch.float32).contiguous()
+        scale_f32 = (scale if scale.dtype == torch.float32 else scale.to(torch.float32)).contiguous()
         if scale_f32.numel() != n:
             raise RuntimeError(f"scale must hold one value per vector ({n}), got shape {tuple(scale.shape)}")
         native = out_dtype in (torch.float32, torch.float16, torch.bfloat16)
         odt = out_dtype if native else torch.float32
-        out = torch.empty(lead + (d,), dtype=odt, device=data.device)
+        dev = data.device
+        out = torch.empty(lead + (d,), dtype=odt, device=dev)
         epl = min(d, 8)
         codes = _lib.aligned(data, max(1, epl if self.bits == 8 else epl // 2))
-        diag = self._diag(d, data.device)
-        with torch.cuda.device(data.device):
-            _lib.check(_lib.lib().aekv_tq_decode(_lib.ptr(codes), _lib.ptr(scale_f32), n, d, self.bits,
-                                                 _lib.ptr(diag), _lib.ptr(out), _lib.dtype_code(out),
-                                                 _lib.stream_of(data)),
-                       "aekv_tq_decode")
+        diag = self._diag(d, dev)
+        with _lib.on_device(dev):
+            rc = _lib.hot("aekv_tq_decode")(codes.data_ptr(), scale_f32.data_ptr(), n, d, self.bits, diag.data_ptr(),
+                                            out.data_ptr(), _lib.TORCH_TO_AEKV[odt], _lib.raw_stream(dev))
+        _lib.check(rc, "aekv_tq_decode")
         return out if native else out.to(out_dtype)
