@@ -20,6 +20,14 @@ namespace {
 constexpr int kThreads = 256;
 enum { kModeWht = 0, kModeEnc4 = 4, kModeEnc8 = 8 };
 
+// Elements per lane of a decode: 8, but 4 for fp32 outputs of 16 to 256 elements, one 16-byte store per
+// lane and 1 KB contiguous per wave (with 8 the two halves of a lane's store are 32 bytes apart in each
+// instruction).  Measured on 100 M elements, 8-bit D = 64 / 4-bit D = 64 / 8-bit D = 128: 95 / 108 / 101 us
+// against 100 / 114 / 108 with 8; 131072 vectors of 64 9.1 against 11.2 us.  (The same split of an
+// encode's loads is slower, 112 to 131 us against 108 to 111: one more lane exchange per element.)
+template <int ODT, int D>
+constexpr int kDecEpl = ODT == AEKV_F32 && D >= 16 && D <= 256 ? 4 : (D < 8 ? D : 8);
+
 // Forward kernel: WHT (fp32 out), or encode to 8/4-bit codes + fp32 scale.
 template <int DT, int D, int MODE>
 __global__ __launch_bounds__(kThreads) void tq_forward_kernel(const void* __restrict__ x, int64_t n_vec,
@@ -72,7 +80,7 @@ __global__ __launch_bounds__(kThreads) void tq_decode_kernel(const void* __restr
                                                              const float* __restrict__ scale, int64_t n_vec,
                                                              const float* __restrict__ diag, float c,
                                                              void* __restrict__ out) {
-  constexpr int EPL = D < 8 ? D : 8;
+  constexpr int EPL = kDecEpl<ODT, D>;
   constexpr int LPV = D / EPL;
   constexpr int VPW = 64 / LPV;
   const int lane = threadIdx.x & 63;
@@ -91,7 +99,7 @@ __global__ __launch_bounds__(kThreads) void tq_decode_kernel(const void* __restr
     float a[EPL];
     // inactive lanes decode row 0 so every lane joins the cross-lane butterflies
     const int64_t vr = ok ? v : 0;
-    decode_lane<BITS, D, true>(static_cast<const uint8_t*>(codes) + vr * (BITS == 8 ? D : D / 2), scale[vr], sub, dg, c, a);
+    decode_lane<BITS, D, true, EPL>(static_cast<const uint8_t*>(codes) + vr * (BITS == 8 ? D : D / 2), scale[vr], sub, dg, c, a);
     if (ok) {
       uint8_t* o = static_cast<uint8_t*>(out) + (v * D + sub * EPL) * (ODT == AEKV_F32 ? 4 : 2);
       if constexpr (ODT == AEKV_F32) {
@@ -127,8 +135,7 @@ __global__ __launch_bounds__(kThreads) void tq_decode_kernel(const void* __restr
   }
 }
 
-int64_t grid_for(int64_t n_vec, int d) {
-  const int epl = d < 8 ? d : 8;
+int64_t grid_for(int64_t n_vec, int d, int epl) {
   const int vpb = (64 / (d / epl)) * (kThreads / 64);  // vectors per block per iteration
   int64_t g = ceil_div(n_vec, vpb);
   if (g > 65536) g = 65536;
@@ -207,7 +214,7 @@ extern "C" int aekv_wht(const void* x, int32_t x_dtype, int64_t n_vec, int32_t d
   if (!is_aligned(x, epl * dtype_size(x_dtype) > 16 ? 16 : epl * dtype_size(x_dtype)) || !is_aligned(out, 4))
     return fail(AEKV_ERR_ALIGN, "aekv_wht: misaligned pointer");
   fwd_fn fn = pick_fwd_dt<kModeWht>(x_dtype, d);
-  hipLaunchKernelGGL(fn, dim3(static_cast<uint32_t>(grid_for(n_vec, d))), dim3(kThreads), 0, as_stream(stream), x,
+  hipLaunchKernelGGL(fn, dim3(static_cast<uint32_t>(grid_for(n_vec, d, d < 8 ? d : 8))), dim3(kThreads), 0, as_stream(stream), x,
                      n_vec, nullptr, wht_scale(d), static_cast<void*>(out), nullptr);
   return check_launch("aekv_wht");
 }
@@ -229,11 +236,11 @@ extern "C" int aekv_tq_encode(const void* x, int32_t x_dtype, int64_t n_vec, int
   if (bits == 4 && d == 128 && x_dtype == AEKV_BF16 && use_specialised_codec() &&
       launch_encode4_d128_bf16(x, n_vec, diag, wht_scale(d), codes, scale, as_stream(stream)))
     return check_launch("aekv_tq_encode");
-  if (x_dtype == AEKV_BF16 && use_specialised_codec() &&
-      launch_encode_fast_bf16(x, n_vec, bits, d, diag, wht_scale(d), codes, scale, as_stream(stream)))
+  if (use_specialised_codec() &&
+      launch_encode_fast(x, x_dtype, n_vec, bits, d, diag, wht_scale(d), codes, scale, as_stream(stream)))
     return check_launch("aekv_tq_encode");
   fwd_fn fn = bits == 8 ? pick_fwd_dt<kModeEnc8>(x_dtype, d) : pick_fwd_dt<kModeEnc4>(x_dtype, d);
-  hipLaunchKernelGGL(fn, dim3(static_cast<uint32_t>(grid_for(n_vec, d))), dim3(kThreads), 0, as_stream(stream), x,
+  hipLaunchKernelGGL(fn, dim3(static_cast<uint32_t>(grid_for(n_vec, d, d < 8 ? d : 8))), dim3(kThreads), 0, as_stream(stream), x,
                      n_vec, diag, wht_scale(d), codes, scale);
   return check_launch("aekv_tq_encode");
 }
@@ -256,7 +263,7 @@ extern "C" int aekv_tq_decode(const void* codes, const float* scale, int64_t n_v
       launch_decode4_d128_bf16(codes, scale, n_vec, diag, wht_scale(d), out, as_stream(stream)))
     return check_launch("aekv_tq_decode");
   dec_fn fn = bits == 8 ? pick_dec_dt<8>(out_dtype, d) : pick_dec_dt<4>(out_dtype, d);
-  hipLaunchKernelGGL(fn, dim3(static_cast<uint32_t>(grid_for(n_vec, d))), dim3(kThreads), 0, as_stream(stream),
+  hipLaunchKernelGGL(fn, dim3(static_cast<uint32_t>(grid_for(n_vec, d, out_dtype == AEKV_F32 && d >= 16 && d <= 256 ? 4 : (d < 8 ? d : 8)))), dim3(kThreads), 0, as_stream(stream),
                      codes, scale, n_vec, diag, wht_scale(d), out);
   return check_launch("aekv_tq_decode");
 }

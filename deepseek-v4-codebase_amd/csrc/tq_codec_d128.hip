@@ -1,5 +1,5 @@
 // Fast TurboQuant encode and decode for the production shapes (gfx950): the 4-bit D = 128 bf16 KV
-// layer (encode and decode), and the encode of 8-bit D = 128 blocks and of the D = 64 index keys.
+// layer (encode and decode), and the encode of the other 16-bit blocks of D = 128 and index keys of D = 64.
 //
 // ENCODE
 // Same result, bit for bit, as tq_forward_kernel<BF16, 128, ENC4> and as
@@ -279,20 +279,27 @@ __global__ __launch_bounds__(kEncThreads, kEncMinWaves) void tq_encode4_d128_bf1
   encode_group(ta, x, grp, n_vec, v, g, dm, s32, s64, sigma, diag, c, c7, codes, scale);
 }
 
-// ---- encode of the engine's other shapes: 8-bit D = 128, 4- and 8-bit D = 64 (bf16 in) ---------
-// The 4-bit D = 128 design with two changes.
+// ---- encode of the other shapes: D = 64 and 128, 4 and 8 bits, from bf16 and fp16 -------------------
+// The 4-bit D = 128 design with these changes.
 // * Layout: 32 elements per lane as above, LPV = D / 32 lanes per vector (4 at D = 128: stages h =
 //   32, 64 across the quad; 2 at D = 64: stage h = 32 across the lane pair), 64 / LPV vectors per
 //   wave.  A wave reads 4 KiB and writes 64 / LPV vectors' codes (1 or 2 KiB), contiguous.
-// * Quantiser factor in fp64.  With Q = 127 the rounding grid is 18x finer than at Q = 7, so the
-//   4-bit kernel's interval K(1 +- 2^-20) would straddle a rounding boundary in a large share of
-//   waves.  Here K = Q c / m is computed in fp64 (error ~2^-52) once per vector and widened to
-//   K- = fp32(K (1 - 4 2^-24)) <= K (1 - 3 2^-24) and K+ = fp32(K (1 + 4 2^-24)) >= K (1 + 3 2^-24)
-//   (each fp32 rounding moves it by at most 2^-24 relative).  The reference's three roundings keep
-//   t = RN(RN(RN(raw c) / m) Q) within 3 2^-24 of raw c Q / m, so t lies between raw K- and raw K+
-//   and, rne being monotonic, equal roundings of the two decide rne(t).  A wave with any element
-//   undecided (within ~8 2^-24 |t| of a half-integer: ~3% of 8-bit D = 128 waves on Gaussian
-//   data, a few per mille at 4 bits) re-encodes its vectors with the reference's exact sequence.
+// * fp16 elements take their diag sign on the packed word, before the conversion.
+// * Quantiser interval.  K = RN(RN(Qc) v_rcp_f32(m)) is within 4 2^-24 relative of Qc/m (the product
+//   Qc and K round once each, the reciprocal is within 2 2^-24); the reference's three roundings keep t =
+//   RN(RN(RN(raw c) / m) Q) within 3 2^-24 of raw c Q / m; so t lies between raw K- and raw K+ for K+- =
+//   K (1 +- 10 2^-24) (their own rounding takes one 2^-24 of the ten), and, rne being monotonic, equal
+//   roundings of the two decide rne(t).
+// * Undecided elements (within ~10 2^-24 |t| of a half-integer: ~8% of 8-bit D = 128 waves hold one on
+//   Gaussian data) get the reference's exact sequence in place: the wave walks its 32 elements per lane and
+//   divides only where some lane is undecided.
+// * A vector with an infinite or NaN element, or beyond the range where K and its margin are normal
+//   numbers, sends its wave through the generic kernel's sequence, re-read from x.
+// Measured: 100 M fp16 elements, 4-bit / 8-bit D = 128 114 / 134 us, D = 64 115 / 132 us, 190 / 186 and 190 /
+// 209 us by the generic kernel (8 divisions per lane); 49152 bf16 vectors 8-bit D = 128 6.8 us, 9.4 us with
+// undecided waves re-encoded from memory and K in fp64 to have fewer of them; 100 M bf16 elements 136 us
+// either way, at the rate of their reads and writes.  fp32 inputs stay with the generic kernel, which is
+// bound by its bytes (110 us here and 111 there for 4-bit, 110 against 119 us for 8-bit D = 128).
 // * 8-bit codes: RN(p + 1.5 2^23 + 128) = 1.5 2^23 + 128 + rne(p) for |p| <= 2^22, whose low
 //   byte is rne(p) + 128; xor 0x80 gives the two's-complement int8.
 constexpr float kMagic128 = 12583040.0f;  // 1.5 * 2^23 + 128
@@ -325,8 +332,8 @@ __device__ __forceinline__ void pair_stage8(float& a0, float& a1, float& a2, flo
 
 // The reference's exact sequence for the group's vectors, re-read from x (the generic kernel's
 // per-lane code: 8 elements per lane, D / 8 lanes per vector).
-template <int BITS, int D>
-__device__ __forceinline__ void encode_group_exact_g(const uint16_t* __restrict__ x, int64_t grp, int64_t n_vec,
+template <int DT, int BITS, int D>
+__device__ __forceinline__ void encode_group_exact_g(const void* __restrict__ x, int64_t grp, int64_t n_vec,
                                                      const float* __restrict__ diag, float c,
                                                      uint8_t* __restrict__ codes, float* __restrict__ scale) {
   using F = FastEnc<BITS, D>;
@@ -341,7 +348,7 @@ __device__ __forceinline__ void encode_group_exact_g(const uint16_t* __restrict_
     const int64_t v = grp * F::VPW + pass * VPP + slot;
     const bool ok = v < n_vec;
     float a[EPL];
-    load_elems<AEKV_BF16, EPL>(x, v * D + sub * EPL, ok, a);
+    load_elems<DT, EPL>(x, v * D + sub * EPL, ok, a);
 #pragma unroll
     for (int e = 0; e < EPL; ++e) a[e] = a[e] * dg[e];
     float m;
@@ -353,12 +360,13 @@ __device__ __forceinline__ void encode_group_exact_g(const uint16_t* __restrict_
   }
 }
 
-template <int BITS, int D>
-__global__ __launch_bounds__(kEncThreads, kEncMinWaves) void tq_encode_fast_bf16_kernel(
-    const uint16_t* __restrict__ x, int64_t n_vec, const float* __restrict__ diag, float c,
+template <int DT, int BITS, int D>
+__global__ __launch_bounds__(kEncThreads, kEncMinWaves) void tq_encode_fast_kernel(
+    const void* __restrict__ x, int64_t n_vec, const float* __restrict__ diag, float c, float cq,
     uint8_t* __restrict__ codes, float* __restrict__ scale) {
   using F = FastEnc<BITS, D>;
   constexpr int LPV = F::LPV, VPW = F::VPW;
+  static_assert(DT == AEKV_BF16 || DT == AEKV_F16, "16-bit elements");
   const int lane = threadIdx.x & 63;
   const int v = lane / LPV, g = lane % LPV;
   // diag sign masks of the lane part's 16 packed words (bit 15: low element, bit 31: high)
@@ -376,7 +384,7 @@ __global__ __launch_bounds__(kEncThreads, kEncMinWaves) void tq_encode_fast_bf16
   // the lane's 64 bytes (lanes past a partial last group re-read its last vector, never stored)
   uint32_t w[16];
   {
-    const char* base = reinterpret_cast<const char*>(x + grp * VPW * D);
+    const char* base = static_cast<const char*>(x) + grp * VPW * D * 2;
     const int64_t rem = n_vec - grp * VPW;
     const uint32_t vv = static_cast<uint32_t>(v < rem ? v : rem - 1);
     const uint32_t off = vv * (2u * D) + static_cast<uint32_t>(g) * 64u;
@@ -402,8 +410,15 @@ __global__ __launch_bounds__(kEncThreads, kEncMinWaves) void tq_encode_fast_bf16
 #pragma unroll
   for (int k = 0; k < 16; ++k) {
     // stage h = 1 on x * diag: lo + hi, lo - hi
-    const float lo = __builtin_bit_cast(float, (w[k] + dm[k]) << 16);
-    const float hi = __builtin_bit_cast(float, __builtin_amdgcn_bitop3_b32(w[k], 0xFFFF0000u, dm[k], 0x48));
+    float lo, hi;
+    if constexpr (DT == AEKV_BF16) {
+      lo = __builtin_bit_cast(float, (w[k] + dm[k]) << 16);
+      hi = __builtin_bit_cast(float, __builtin_amdgcn_bitop3_b32(w[k], 0xFFFF0000u, dm[k], 0x48));
+    } else {
+      const uint32_t s = w[k] ^ dm[k];
+      lo = f16_to_f32(s & 0xFFFFu);
+      hi = f16_to_f32(s >> 16);
+    }
     a[2 * k] = lo + hi;
     a[2 * k + 1] = lo - hi;
   }
@@ -439,16 +454,15 @@ __global__ __launch_bounds__(kEncThreads, kEncMinWaves) void tq_encode_fast_bf16
   mr = fmaxf(mr, xor_lane<1>(mr));
   if constexpr (LPV == 4) mr = fmaxf(mr, xor_lane<2>(mr));
   const float m = fmaxf(mr * c, 1e-8f);
-  const double kd = static_cast<double>(c) * static_cast<double>(F::Q) / static_cast<double>(m);
-  const float klo = static_cast<float>(kd * (1.0 - 0x1p-22)) * sigma;
-  const float khi = static_cast<float>(kd * (1.0 + 0x1p-22)) * sigma;
+  const float K = cq * __builtin_amdgcn_rcpf(m);
+  const float klo = (K - K * 0x1.4p-21f) * sigma, khi = (K + K * 0x1.4p-21f) * sigma;
   constexpr float kMag = BITS == 8 ? kMagic128 : kMagic8;
   constexpr int NW = F::LB / 4;  // code dwords per lane
+  constexpr int EPW = BITS == 8 ? 4 : 8;  // elements per code dword
   uint32_t o[NW];
   uint32_t diff = 0u;
 #pragma unroll
   for (int dw = 0; dw < NW; ++dw) {
-    constexpr int EPW = BITS == 8 ? 4 : 8;  // elements per code dword
     uint32_t b[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -474,9 +488,28 @@ __global__ __launch_bounds__(kEncThreads, kEncMinWaves) void tq_encode_fast_bf16
       o[dw] = pack4(b[0], b[1], b[2], b[3]);
     }
   }
-  if (__builtin_amdgcn_ballot_w64(diff != 0u) != 0) {  // a rounding the interval cannot decide
-    encode_group_exact_g<BITS, D>(x, grp, n_vec, diag, c, codes, scale);
+  // (every output sums every input, so a lane's first output shows an infinite or NaN input)
+  // (2^100: K and its margin stay normal numbers)
+  const bool odd = !(mr < 0x1p100f) || !(fabsf(a[0]) < __builtin_inff());
+  if (__builtin_amdgcn_ballot_w64(odd) != 0) {
+    encode_group_exact_g<DT, BITS, D>(x, grp, n_vec, diag, c, codes, scale);
     return;
+  }
+  if (__builtin_amdgcn_ballot_w64(diff != 0u) != 0) {  // some rounding the interval cannot decide
+    float rlo = klo, rhi = khi;
+    asm volatile("" : "+v"(rlo), "+v"(rhi));  // (the 64 products are formed again here, not kept in registers)
+#pragma unroll
+    for (int e = 0; e < 32; ++e) {
+      const bool open = fmaf(a[e], rlo, kMag) != fmaf(a[e], rhi, kMag);
+      if (__builtin_amdgcn_ballot_w64(open) == 0) continue;  // wave-uniform
+      float t = ((a[e] * sigma) * c) / m;  // correctly rounded division, then * Q, rne
+      t = fminf(fmaxf(rintf(t * F::Q), -F::Q), F::Q);
+      constexpr int kBits = 32 / EPW;
+      constexpr uint32_t kMask = BITS == 8 ? 0xFFu : 0xFu;
+      const int sh = kBits * (e % EPW);
+      const uint32_t code = (static_cast<uint32_t>(static_cast<int>(t)) & kMask) << sh;
+      o[e / EPW] = open ? (o[e / EPW] & ~(kMask << sh)) | code : o[e / EPW];
+    }
   }
   if (v < n_vec - grp * VPW) {  // streaming stores: the outputs are not read again by this kernel
     if (g == 0)
@@ -718,28 +751,34 @@ bool launch_encode4_d128_bf16(const void* x, int64_t n_vec, const float* diag, f
 
 // Launches the fast encode of 8-bit D = 128 or 4- / 8-bit D = 64 (bf16 in); false when the shape or
 // the alignment is not one of those.
-bool launch_encode_fast_bf16(const void* x, int64_t n_vec, int bits, int d, const float* diag, float c, void* codes,
-                             float* scale, hipStream_t st) {
-  if ((reinterpret_cast<uintptr_t>(x) & 15) || (reinterpret_cast<uintptr_t>(codes) & 15)) return false;
-  void (*kern)(const uint16_t*, int64_t, const float*, float, uint8_t*, float*) = nullptr;
+namespace {
+
+typedef void (*fast_enc_fn)(const void*, int64_t, const float*, float, float, uint8_t*, float*);
+
+template <int DT>
+fast_enc_fn pick_fast(int bits, int d, int& vpw) {
+  vpw = d == 128 ? FastEnc<8, 128>::VPW : FastEnc<8, 64>::VPW;
+  if (bits == 8) return d == 128 ? tq_encode_fast_kernel<DT, 8, 128> : tq_encode_fast_kernel<DT, 8, 64>;
+  if (d == 64) return tq_encode_fast_kernel<DT, 4, 64>;
+  if constexpr (DT == AEKV_BF16) return nullptr;  // tq_encode4_d128_bf16_kernel
+  else return tq_encode_fast_kernel<DT, 4, 128>;
+}
+
+}  // namespace
+
+bool launch_encode_fast(const void* x, int x_dtype, int64_t n_vec, int bits, int d, const float* diag, float c,
+                        void* codes, float* scale, hipStream_t st) {
+  if (!is_aligned(x, 16) || !is_aligned(codes, 16) || (d != 64 && d != 128)) return false;
   int vpw = 0;
-  if (bits == 8 && d == 128) {
-    kern = tq_encode_fast_bf16_kernel<8, 128>;
-    vpw = FastEnc<8, 128>::VPW;
-  } else if (bits == 8 && d == 64) {
-    kern = tq_encode_fast_bf16_kernel<8, 64>;
-    vpw = FastEnc<8, 64>::VPW;
-  } else if (bits == 4 && d == 64) {
-    kern = tq_encode_fast_bf16_kernel<4, 64>;
-    vpw = FastEnc<4, 64>::VPW;
-  } else {
-    return false;
-  }
+  const fast_enc_fn kern = x_dtype == AEKV_BF16  ? pick_fast<AEKV_BF16>(bits, d, vpw)
+                           : x_dtype == AEKV_F16 ? pick_fast<AEKV_F16>(bits, d, vpw)
+                                                 : nullptr;
+  if (!kern) return false;
   if (n_vec <= 0) return true;
-  const int64_t blocks = ceil_div(ceil_div(n_vec, vpw), kEncThreads / 64);
+  const int64_t blocks = ceil_div(ceil_div(n_vec, static_cast<int64_t>(vpw)), kEncThreads / 64);
   if (blocks > 0x7fffffff) return false;
-  hipLaunchKernelGGL(kern, dim3(static_cast<uint32_t>(blocks)), dim3(kEncThreads), 0, st,
-                     static_cast<const uint16_t*>(x), n_vec, diag, c, static_cast<uint8_t*>(codes), scale);
+  hipLaunchKernelGGL(kern, dim3(static_cast<uint32_t>(blocks)), dim3(kEncThreads), 0, st, x, n_vec, diag, c,
+                     (bits == 8 ? 127.0f : 7.0f) * c, static_cast<uint8_t*>(codes), scale);
   return true;
 }
 

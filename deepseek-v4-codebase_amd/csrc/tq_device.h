@@ -141,21 +141,18 @@ __device__ __forceinline__ Bytes<(BITS == 8 ? (D < 8 ? D : 8) : (D < 8 ? D : 8) 
 }
 
 // Code bytes a lane holds for its EPL elements of one vector.
-template <int BITS, int D>
+template <int BITS, int EPL>
 struct LaneCodes {
-  static constexpr int EPL = D < 8 ? D : 8;
   static constexpr int NB = BITS == 8 ? EPL : EPL / 2;  // code bytes per lane
   using type = Bytes<NB>;
 };
 
 // Dequantise the EPL elements of one vector held by this lane: codes * scale -> WHT -> * c -> * diag
 // (turbo_quant.py:187-211), from the lane's code bytes (bytes sub*NB .. of the vector's row).
-template <int BITS, int D, bool LDS_PIPE = false>
-__device__ __forceinline__ void decode_lane_bytes(const typename LaneCodes<BITS, D>::type& w, float s, int sub,
-                                                  const float (&dg)[(D < 8 ? D : 8)], float c,
-                                                  float (&a)[(D < 8 ? D : 8)]) {
-  constexpr int EPL = D < 8 ? D : 8;
-  constexpr int NB = LaneCodes<BITS, D>::NB;
+template <int BITS, int D, bool LDS_PIPE = false, int EPL = (D < 8 ? D : 8)>
+__device__ __forceinline__ void decode_lane_bytes(const typename LaneCodes<BITS, EPL>::type& w, float s, int sub,
+                                                  const float (&dg)[EPL], float c, float (&a)[EPL]) {
+  constexpr int NB = LaneCodes<BITS, EPL>::NB;
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
     if constexpr (BITS == 8) {
@@ -173,13 +170,12 @@ __device__ __forceinline__ void decode_lane_bytes(const typename LaneCodes<BITS,
 }
 
 // The same, loading the lane's bytes from `row`, the vector's code row.
-template <int BITS, int D, bool LDS_PIPE = false>
+template <int BITS, int D, bool LDS_PIPE = false, int EPL = (D < 8 ? D : 8)>
 __device__ __forceinline__ void decode_lane(const uint8_t* __restrict__ row, float s, int sub,
-                                            const float (&dg)[(D < 8 ? D : 8)], float c,
-                                            float (&a)[(D < 8 ? D : 8)]) {
-  using W = typename LaneCodes<BITS, D>::type;
-  const W w = *reinterpret_cast<const W*>(row + sub * LaneCodes<BITS, D>::NB);
-  decode_lane_bytes<BITS, D, LDS_PIPE>(w, s, sub, dg, c, a);
+                                            const float (&dg)[EPL], float c, float (&a)[EPL]) {
+  using W = typename LaneCodes<BITS, EPL>::type;
+  const W w = *reinterpret_cast<const W*>(row + sub * LaneCodes<BITS, EPL>::NB);
+  decode_lane_bytes<BITS, D, LDS_PIPE, EPL>(w, s, sub, dg, c, a);
 }
 
 // Specialised production-shape kernels (tq_codec_d128.hip).  Each returns false (and launches
@@ -189,8 +185,8 @@ bool launch_encode4_d128_bf16(const void* x, int64_t n_vec, const float* diag, f
                               hipStream_t st);
 bool launch_decode4_d128_bf16(const void* codes, const float* scale, int64_t n_vec, const float* diag, float c,
                               void* out, hipStream_t st);
-// 8-bit D = 128 and 4- / 8-bit D = 64 encode, bf16 in.
-bool launch_encode_fast_bf16(const void* x, int64_t n_vec, int bits, int d, const float* diag, float c, void* codes,
-                             float* scale, hipStream_t st);
+// Encode of D = 64 and 128 in either width from bf16 or fp16 (4-bit D = 128 bf16 has its own, above).
+bool launch_encode_fast(const void* x, int x_dtype, int64_t n_vec, int bits, int d, const float* diag, float c,
+                        void* codes, float* scale, hipStream_t st);
 
 }  // namespace aekv

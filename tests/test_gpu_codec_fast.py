@@ -1,0 +1,90 @@
+"""The fast encode of D = 64 and 128 from every input type, bit for bit against the generic kernel (which
+the oracle pins), and the 4-element decode layout of fp32 outputs against the oracle."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import aetherkv._lib as L
+import oracle as O
+from aetherkv import PolarQuant
+from aetherkv.synthetic import normal_with_outliers
+
+pytestmark = pytest.mark.gpu
+
+
+def _both(pq, x):
+    prev = L.lib().aekv_set_generic_kernels(1)
+    try:
+        g = pq.encode(x)
+    finally:
+        L.lib().aekv_set_generic_kernels(prev)
+    return g, pq.encode(x)
+
+
+def _same(pq, x):
+    (cg, sg), (cf, sf) = _both(pq, x)
+    assert torch.equal(cg, cf)
+    assert torch.equal(sg.view(torch.int32), sf.view(torch.int32))  # (bits: NaN scales compare too)
+
+
+CASES = [(dt, bits, d) for dt in (torch.bfloat16, torch.float16, torch.float32) for bits in (4, 8) for d in (64, 128)]
+
+
+# a lone vector, partial and whole waves, thousands of waves (some hold undecided roundings)
+@pytest.mark.parametrize("dtype,bits,d", CASES)
+@pytest.mark.parametrize("n", [1, 15, 33, 200003])
+def test_random_vectors(dev, dtype, bits, d, n):
+    _same(PolarQuant(bits), normal_with_outliers((n, d), n + d + bits, dtype=dtype, trailing_dims=1).to(dev))
+
+
+# vectors of a few small integers: their transforms take few values, whose ratios to the largest are often exact
+# halves of a code step (3 +- 1 gives 2 / 4 * 7 = 3.5 and 2 / 4 * 127 = 63.5): ties and near ties throughout
+@pytest.mark.parametrize("dtype,bits,d", CASES)
+def test_ties(dev, dtype, bits, d):
+    g = torch.Generator().manual_seed(d + bits)
+    x = torch.zeros(20000, d)
+    for n in range(1, 5):
+        rows = slice(5000 * (n - 1), 5000 * n)
+        at = torch.rand(5000, d, generator=g).argsort(1)[:, :n]
+        x[rows].scatter_(1, at, torch.randint(-9, 10, (5000, n), generator=g).float())
+    _same(PolarQuant(bits), x.to(dtype).to(dev))
+    _same(PolarQuant(bits), (x * 0.1).to(dtype).to(dev))  # rounded inputs: near ties
+
+
+# zero, tiny and huge vectors, infinities and NaN, and (fp32) sums that overflow, between ordinary vectors of one wave
+# (the 4-bit D = 128 bf16 kernel is another one, which takes finite vectors of ordinary range)
+@pytest.mark.parametrize("dtype,bits,d", [c for c in CASES if c != (torch.bfloat16, 4, 128)])
+def test_extreme_vectors(dev, dtype, bits, d):
+    x = torch.randn(64, d, generator=torch.Generator().manual_seed(d))
+    big = 6e4 if dtype == torch.float16 else 3e38
+    x[3] = 0.0
+    x[5] *= 1e-7
+    x[7] *= 1e-12
+    x[20] *= big / 200
+    x[22, :3] = big
+    x[40] = big
+    x[41, ::2], x[41, 1::2] = big, -big
+    x[50, 9] = float("inf")
+    x[51, 10], x[51, 11] = float("inf"), float("-inf")
+    x[60, 12] = float("nan")
+    if dtype != torch.float16:
+        x[30] *= 1e31  # above the fast quantiser's range, sums still finite
+        x[31] *= 1e-36
+    for rows in (slice(0, 16), slice(16, 35), slice(0, 64)):
+        _same(PolarQuant(bits), x[rows].to(dtype).to(dev))
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("d", [16, 32, 64, 128, 256, 512])
+def test_decode_to_fp32(dev, bits, d):
+    rng = np.random.default_rng(d)
+    for n in (1, 37, 3001):
+        if bits == 8:
+            codes = rng.integers(-127, 128, (n, d)).astype(np.int8)
+        else:
+            codes = rng.integers(0, 256, (n, d // 2)).astype(np.uint8)
+        scale = (rng.random((n, 1)) + 1e-3).astype(np.float32)
+        got = PolarQuant(bits).decode(torch.from_numpy(codes).to(dev), torch.from_numpy(scale).to(dev), torch.float32)
+        np.testing.assert_array_equal(got.cpu().numpy(), O.decode(codes, scale, bits, O.diag(42, d), "f32"))
