@@ -97,7 +97,7 @@ __global__ __launch_bounds__(NT) void sink_attn_combine_kernel(const float* __re
     float cm = M;
 #pragma unroll
     for (int i = 0; i < kChunk; ++i) cm = fmaxf(cm, m[i]);
-    if (cm == kNegInf) continue;  // nothing yet (no sink, no source)
+    // (nothing yet, no sink and no source: the sums stay zero, or NaN where a piece's are)
     const float r = M == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(M - cm);
     den *= r;
     acc *= r;

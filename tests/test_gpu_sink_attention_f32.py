@@ -92,3 +92,14 @@ def test_unsplit_and_small_workspace_agree(dev):
     for out in outs:
         _check(out, q, kv, np.broadcast_to(np.arange(S), (B, T, S)), sink, D ** -0.5)
     assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("K", [50, 1500])  # whole, and split into pieces
+def test_no_sink_and_no_maximum(dev, K):
+    # a sink of -inf leaves a target without sources at zero, and one whose logits are all NaN at NaN
+    g, q, kv, _ = _inputs(11, 1, 2, 12, 128, 900, torch.float32)
+    q[0, 1] = float("nan")
+    idx = torch.randint(0, 900, (1, 2, K), generator=g)
+    idx[0, 0] = -1
+    got = sparse_sink_attention(q.to(dev), kv.to(dev), idx.to(dev), torch.full((12,), float("-inf"), device=dev), 128 ** -0.5)
+    assert bool((got[0, 0] == 0).all()) and bool(torch.isnan(got[0, 1]).all())
