@@ -74,8 +74,41 @@ __global__ __launch_bounds__(kThreads) void tq_forward_kernel(const void* __rest
   }
 }
 
-// Decode kernel: codes * scale -> WHT -> * diag -> out dtype.
-template <int BITS, int D, int ODT>
+// Stores a lane's EPL decoded elements at o, rounded to ODT; NT: past the caches.
+template <int ODT, int EPL, bool NT>
+__device__ __forceinline__ void store_decoded(uint8_t* o, const float (&a)[EPL]) {
+  constexpr int NB = EPL * (ODT == AEKV_F32 ? 4 : 2);
+  Bytes<NB> w;
+  if constexpr (ODT == AEKV_F32) {
+    __builtin_memcpy(w.b, a, NB);
+  } else if constexpr (ODT == AEKV_BF16 && EPL >= 2) {
+    uint32_t wv[EPL / 2];
+#pragma unroll
+    for (int i = 0; i < EPL / 2; ++i) wv[i] = pack_bf16x2(a[2 * i], a[2 * i + 1]);
+    __builtin_memcpy(w.b, wv, NB);
+  } else {
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) {
+      const uint16_t h = static_cast<uint16_t>(ODT == AEKV_BF16 ? pack_bf16x2(a[e], 0.0f) & 0xffffu : f32_to_f16_bits(a[e]));
+      __builtin_memcpy(w.b + 2 * e, &h, 2);
+    }
+  }
+  if constexpr (NT) {
+    static_assert(NB == 16, "one 16-byte store per lane");
+    typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
+    __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, w), reinterpret_cast<u32x4_t*>(o));
+  } else if constexpr (NB <= 16) {
+    *reinterpret_cast<Bytes<NB>*>(o) = w;
+  } else {
+    reinterpret_cast<Bytes<16>*>(o)[0] = *reinterpret_cast<Bytes<16>*>(w.b);
+    reinterpret_cast<Bytes<16>*>(o)[1] = *reinterpret_cast<Bytes<16>*>(w.b + 16);
+  }
+}
+
+// Decode kernel: codes * scale -> WHT -> * diag -> out dtype.  PP == 0: a grid-stride loop.  PP > 0: PP
+// consecutive groups of 64 / LPV vectors per wave, all their loads issued first, no loop (the launch covers
+// every group), and stores past the caches.
+template <int BITS, int D, int ODT, int PP>
 __global__ __launch_bounds__(kThreads) void tq_decode_kernel(const void* __restrict__ codes,
                                                              const float* __restrict__ scale, int64_t n_vec,
                                                              const float* __restrict__ diag, float c,
@@ -83,15 +116,37 @@ __global__ __launch_bounds__(kThreads) void tq_decode_kernel(const void* __restr
   constexpr int EPL = kDecEpl<ODT, D>;
   constexpr int LPV = D / EPL;
   constexpr int VPW = 64 / LPV;
+  constexpr int RB = BITS == 8 ? D : D / 2, OB = D * (ODT == AEKV_F32 ? 4 : 2);  // bytes of a vector
   const int lane = threadIdx.x & 63;
   const int sub = lane % LPV;
   const int slot = lane / LPV;
+  const uint8_t* cb = static_cast<const uint8_t*>(codes);
+  uint8_t* ob = static_cast<uint8_t*>(out) + sub * (OB / LPV);
 
   float dg[EPL];
 #pragma unroll
   for (int e = 0; e < EPL; ++e) dg[e] = diag[sub * EPL + e];
 
   const int64_t wave = (static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x) >> 6;
+  if constexpr (PP > 0) {
+    using LC = LaneCodes<BITS, EPL>;
+    const int64_t v0 = wave * (PP * VPW) + slot;
+    typename LC::type w[PP];
+    float s[PP];
+#pragma unroll
+    for (int i = 0; i < PP; ++i) {  // (lanes past the end decode row 0, never stored)
+      const int64_t v = v0 + i * VPW, vr = v < n_vec ? v : 0;
+      w[i] = *reinterpret_cast<const typename LC::type*>(cb + vr * RB + sub * LC::NB);
+      s[i] = scale[vr];
+    }
+#pragma unroll
+    for (int i = 0; i < PP; ++i) {
+      float a[EPL];
+      decode_lane_bytes<BITS, D, true, EPL>(w[i], s[i], sub, dg, c, a);
+      if (v0 + i * VPW < n_vec) store_decoded<ODT, EPL, true>(ob + (v0 + i * VPW) * OB, a);
+    }
+    return;
+  }
   const int64_t n_waves = (static_cast<int64_t>(gridDim.x) * kThreads) >> 6;
   for (int64_t base = wave * VPW; base < n_vec; base += n_waves * VPW) {
     const int64_t v = base + slot;
@@ -99,39 +154,8 @@ __global__ __launch_bounds__(kThreads) void tq_decode_kernel(const void* __restr
     float a[EPL];
     // inactive lanes decode row 0 so every lane joins the cross-lane butterflies
     const int64_t vr = ok ? v : 0;
-    decode_lane<BITS, D, true, EPL>(static_cast<const uint8_t*>(codes) + vr * (BITS == 8 ? D : D / 2), scale[vr], sub, dg, c, a);
-    if (ok) {
-      uint8_t* o = static_cast<uint8_t*>(out) + (v * D + sub * EPL) * (ODT == AEKV_F32 ? 4 : 2);
-      if constexpr (ODT == AEKV_F32) {
-        Bytes<EPL * 4> w;
-        __builtin_memcpy(w.b, a, EPL * 4);
-        if constexpr (EPL * 4 <= 16) {
-          *reinterpret_cast<Bytes<EPL * 4>*>(o) = w;
-        } else {
-          reinterpret_cast<Bytes<16>*>(o)[0] = *reinterpret_cast<Bytes<16>*>(w.b);
-          reinterpret_cast<Bytes<16>*>(o)[1] = *reinterpret_cast<Bytes<16>*>(w.b + 16);
-        }
-      } else if constexpr (ODT == AEKV_BF16) {
-        if constexpr (EPL >= 2) {
-          uint32_t wv[EPL / 2];
-#pragma unroll
-          for (int i = 0; i < EPL / 2; ++i) wv[i] = pack_bf16x2(a[2 * i], a[2 * i + 1]);
-          Bytes<EPL * 2> w;
-          __builtin_memcpy(w.b, wv, EPL * 2);
-          *reinterpret_cast<Bytes<EPL * 2>*>(o) = w;
-        } else {
-          *reinterpret_cast<uint16_t*>(o) = static_cast<uint16_t>(pack_bf16x2(a[0], 0.0f) & 0xffffu);
-        }
-      } else {
-        Bytes<EPL * 2> w;
-#pragma unroll
-        for (int e = 0; e < EPL; ++e) {
-          const uint16_t h = static_cast<uint16_t>(f32_to_f16_bits(a[e]));
-          __builtin_memcpy(w.b + 2 * e, &h, 2);
-        }
-        *reinterpret_cast<Bytes<EPL * 2>*>(o) = w;
-      }
-    }
+    decode_lane<BITS, D, true, EPL>(cb + vr * RB, scale[vr], sub, dg, c, a);
+    if (ok) store_decoded<ODT, EPL, false>(ob + v * OB, a);
   }
 }
 
@@ -172,18 +196,37 @@ fwd_fn pick_fwd_dt(int dt, int d) {
 template <int BITS, int ODT>
 dec_fn pick_dec(int d) {
   switch (d) {
-    case 1: return BITS == 4 ? nullptr : tq_decode_kernel<BITS, 1, ODT>;
-    case 2: return tq_decode_kernel<BITS, 2, ODT>;
-    case 4: return tq_decode_kernel<BITS, 4, ODT>;
-    case 8: return tq_decode_kernel<BITS, 8, ODT>;
-    case 16: return tq_decode_kernel<BITS, 16, ODT>;
-    case 32: return tq_decode_kernel<BITS, 32, ODT>;
-    case 64: return tq_decode_kernel<BITS, 64, ODT>;
-    case 128: return tq_decode_kernel<BITS, 128, ODT>;
-    case 256: return tq_decode_kernel<BITS, 256, ODT>;
-    case 512: return tq_decode_kernel<BITS, 512, ODT>;
+    case 1: return BITS == 4 ? nullptr : tq_decode_kernel<BITS, 1, ODT, 0>;
+    case 2: return tq_decode_kernel<BITS, 2, ODT, 0>;
+    case 4: return tq_decode_kernel<BITS, 4, ODT, 0>;
+    case 8: return tq_decode_kernel<BITS, 8, ODT, 0>;
+    case 16: return tq_decode_kernel<BITS, 16, ODT, 0>;
+    case 32: return tq_decode_kernel<BITS, 32, ODT, 0>;
+    case 64: return tq_decode_kernel<BITS, 64, ODT, 0>;
+    case 128: return tq_decode_kernel<BITS, 128, ODT, 0>;
+    case 256: return tq_decode_kernel<BITS, 256, ODT, 0>;
+    case 512: return tq_decode_kernel<BITS, 512, ODT, 0>;
     default: return nullptr;
   }
+}
+
+constexpr int kDecPasses = 4;
+// Codes and output together from which a decode streams (D = 64 and 128).  Measured, loop / streamed, on codes
+// coming round from three sets: 64 M elements to fp32 74 to 80 / 45 to 49 us (8-bit D = 64: 4.6 / 7.0 TB/s), 64 M
+// to bf16 8-bit 39 to 40 / 31, 100 M to fp16 60 to 66 / 46 to 54, 403 M to bf16 8-bit D = 64 234 / 207; 32 M to
+// fp32 (151 to 168 MB) 24 to 27 / 25 to 28, below that within the noise: the loop's output then stays in the caches.
+constexpr int64_t kDecStreamBytes = 160000000;
+
+template <int BITS, int ODT>
+dec_fn pick_dec_stream(int d) {
+  return d == 128 ? tq_decode_kernel<BITS, 128, ODT, kDecPasses> : tq_decode_kernel<BITS, 64, ODT, kDecPasses>;
+}
+
+template <int BITS>
+dec_fn pick_dec_stream_dt(int odt, int d) {
+  if (odt == AEKV_F32) return pick_dec_stream<BITS, AEKV_F32>(d);
+  if (odt == AEKV_F16) return pick_dec_stream<BITS, AEKV_F16>(d);
+  return pick_dec_stream<BITS, AEKV_BF16>(d);
 }
 
 template <int BITS>
@@ -262,8 +305,17 @@ extern "C" int aekv_tq_decode(const void* codes, const float* scale, int64_t n_v
   if (bits == 4 && d == 128 && out_dtype == AEKV_BF16 && use_specialised_codec() &&
       launch_decode4_d128_bf16(codes, scale, n_vec, diag, wht_scale(d), out, as_stream(stream)))
     return check_launch("aekv_tq_decode");
+  const int lane_el = out_dtype == AEKV_F32 && d >= 16 && d <= 256 ? 4 : epl;  // kDecEpl
+  const int64_t blocks = ceil_div(n_vec, static_cast<int64_t>(kDecPasses) * (kThreads / 64) * (64 / (d / lane_el)));
+  const int64_t bytes = n_vec * d * static_cast<int64_t>(dtype_size(out_dtype)) + n_vec * d * bits / 8;
+  if (use_specialised_codec() && (d == 64 || d == 128) && bytes >= kDecStreamBytes && blocks <= 0x7fffffff) {
+    dec_fn fn = bits == 8 ? pick_dec_stream_dt<8>(out_dtype, d) : pick_dec_stream_dt<4>(out_dtype, d);
+    hipLaunchKernelGGL(fn, dim3(static_cast<uint32_t>(blocks)), dim3(kThreads), 0, as_stream(stream), codes, scale, n_vec,
+                       diag, wht_scale(d), out);
+    return check_launch("aekv_tq_decode");
+  }
   dec_fn fn = bits == 8 ? pick_dec_dt<8>(out_dtype, d) : pick_dec_dt<4>(out_dtype, d);
-  hipLaunchKernelGGL(fn, dim3(static_cast<uint32_t>(grid_for(n_vec, d, out_dtype == AEKV_F32 && d >= 16 && d <= 256 ? 4 : (d < 8 ? d : 8)))), dim3(kThreads), 0, as_stream(stream),
+  hipLaunchKernelGGL(fn, dim3(static_cast<uint32_t>(grid_for(n_vec, d, lane_el))), dim3(kThreads), 0, as_stream(stream),
                      codes, scale, n_vec, diag, wht_scale(d), out);
   return check_launch("aekv_tq_decode");
 }

@@ -749,8 +749,6 @@ bool launch_encode4_d128_bf16(const void* x, int64_t n_vec, const float* diag, f
 }
 
 
-// Launches the fast encode of 8-bit D = 128 or 4- / 8-bit D = 64 (bf16 in); false when the shape or
-// the alignment is not one of those.
 namespace {
 
 typedef void (*fast_enc_fn)(const void*, int64_t, const float*, float, float, uint8_t*, float*);
@@ -766,6 +764,7 @@ fast_enc_fn pick_fast(int bits, int d, int& vpw) {
 
 }  // namespace
 
+// Launches the fast encode; false when the shape, the type or the alignment is not one of its own.
 bool launch_encode_fast(const void* x, int x_dtype, int64_t n_vec, int bits, int d, const float* diag, float c,
                         void* codes, float* scale, hipStream_t st) {
   if (!is_aligned(x, 16) || !is_aligned(codes, 16) || (d != 64 && d != 128)) return false;

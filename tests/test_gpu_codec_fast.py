@@ -88,3 +88,26 @@ def test_decode_to_fp32(dev, bits, d):
         scale = (rng.random((n, 1)) + 1e-3).astype(np.float32)
         got = PolarQuant(bits).decode(torch.from_numpy(codes).to(dev), torch.from_numpy(scale).to(dev), torch.float32)
         np.testing.assert_array_equal(got.cpu().numpy(), O.decode(codes, scale, bits, O.diag(42, d), "f32"))
+
+
+# decodes past the caches (160 MB of codes and output), with a last wave and group partly filled
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("bits,d", [(4, 64), (8, 64), (4, 128), (8, 128)])
+def test_streamed_decode(dev, dtype, bits, d):
+    es = 4 if dtype == torch.float32 else 2
+    n = -(-160_000_000 // (d * es + d * bits // 8)) + 37
+    g = torch.Generator(device=dev).manual_seed(n + bits)
+    lo, hi = (0, 256) if bits == 4 else (-127, 128)
+    codes = torch.randint(lo, hi, (n, d * bits // 8), generator=g, device=dev, dtype=torch.uint8 if bits == 4 else torch.int8)
+    scale = torch.rand(n, 1, generator=g, device=dev)
+    scale[::1000] = 0.0
+    pq = PolarQuant(bits)
+    got = pq.decode(codes, scale, dtype)
+    prev = L.lib().aekv_set_generic_kernels(1)
+    try:
+        want = pq.decode(codes, scale, dtype)
+    finally:
+        L.lib().aekv_set_generic_kernels(prev)
+    assert torch.equal(got, want)
+    small = pq.decode(codes[-100:], scale[-100:], dtype)  # (below the line)
+    assert torch.equal(small, got[-100:])
