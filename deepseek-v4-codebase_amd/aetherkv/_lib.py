@@ -179,20 +179,22 @@ def on_device(device: torch.device):
 
 
 # Split workspaces of the drop-in attention calls, one per (device, stream): calls on one stream run
-# in order, so each reuses the previous call's buffer.  Not grown while a graph is being captured
-# (the buffer would come from the graph's private pool): such calls get a buffer of their own.
+# in order, so each reuses the previous call's buffer.  A call that is being captured into a graph
+# always gets a buffer of its own, from the graph's private pool: its replays keep the address, while
+# a cached buffer is replaced when a larger call comes and belongs to the eager calls of its stream.
 _ws_cache: dict = {}
 
 
 def workspace(nbytes: int, device: torch.device, stream: int) -> Optional[torch.Tensor]:
+    """A buffer of at least nbytes for a call on `stream`, the current stream of the current device."""
     if nbytes <= 0:
         return None
+    if torch.cuda.is_current_stream_capturing():
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
     key = (device.index, stream)
     buf = _ws_cache.get(key)
     if buf is not None and buf.numel() >= nbytes:
         return buf
-    if torch.cuda.is_current_stream_capturing():
-        return torch.empty(nbytes, dtype=torch.uint8, device=device)
     buf = torch.empty(max(nbytes, 2 * buf.numel() if buf is not None else 0), dtype=torch.uint8, device=device)
     _ws_cache[key] = buf
     return buf

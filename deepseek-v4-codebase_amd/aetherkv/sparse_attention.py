@@ -10,7 +10,8 @@ Reference: aether_kernels/sparse_attention.py:8-83 (wrappers) and aether_kernels
 
 Outputs are freshly allocated tensors on the inputs' device; kernels run on the current stream.  The
 attention calls also take a split workspace when the matrix-core launch would leave most CUs idle
-(few targets, many sources): one buffer per (device, stream), reused by the calls on that stream.
+(few targets, many sources): one buffer per (device, stream), reused by the calls on that stream; a
+call that is captured into a graph takes a buffer of its own from the graph's pool.
 The host-side cost per call is kept small because the reference's callers make one call per target
 token (modeling.py:322,534): pointers go to the library as plain integers, the stream handle is read
 without building a Stream object, the device is switched only when it is not already current, and
@@ -68,8 +69,8 @@ def _ext_sparse_sink_attention(q, kv, topk_indices, sink, softmax_scale):
     if dt is None:
         raise RuntimeError(f"unsupported dtype {q.dtype}")
     st = _lib.raw_stream(dev)
-    ws = _lib.workspace(_ws_bytes(dt, B, T, H, D, S, K), dev, st)
     with _lib.on_device(dev):
+        ws = _lib.workspace(_ws_bytes(dt, B, T, H, D, S, K), dev, st)
         rc = _lib.hot("aekv_sparse_sink_attention_ws")(
             q.data_ptr(), kv.data_ptr(), topk_indices.data_ptr(), _lib.I64 if topk_indices.dtype == torch.int64
             else _lib.I32, sink.data_ptr(), sink.numel(), dt, B, T, H, D, S, K, float(softmax_scale),
@@ -126,8 +127,8 @@ def _ext_tiled_prefill_attention(q, kv, sink, softmax_scale, tile_size):
     if dt is None:
         raise RuntimeError(f"unsupported dtype {q.dtype}")
     st = _lib.raw_stream(dev)
-    ws = _lib.workspace(_ws_bytes(dt, B, T, H, D, S, -1), dev, st)
     with _lib.on_device(dev):
+        ws = _lib.workspace(_ws_bytes(dt, B, T, H, D, S, -1), dev, st)
         rc = _lib.hot("aekv_tiled_prefill_attention_ws")(
             q.data_ptr(), kv.data_ptr(), sink.data_ptr(), sink.numel(), dt, B, T, H, D, S, float(softmax_scale),
             int(tile_size), None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), out.data_ptr(), st)
