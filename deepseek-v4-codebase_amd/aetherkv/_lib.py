@@ -201,7 +201,9 @@ def workspace(nbytes: int, device: torch.device, stream: int) -> Optional[torch.
 
 
 # Workspace sizes that depend on the call's sizes alone, memoised: the calls that use them run once per
-# layer and token.  (The prefill attention's also depends on the device and on aekv_set_flash_rows.)
+# layer and token.  Called with plain ints: a tensor would be a key by its identity, with the size of the
+# value that it held first.  (The prefill attention's also depends on the device and on
+# aekv_set_flash_rows.)
 @functools.lru_cache(maxsize=1024)
 def indexer_ws_bytes(B: int, S: int, k: int) -> int:
     return lib().aekv_csa_indexer_workspace_size(B, S, k)

@@ -100,11 +100,12 @@ def _prefix_rows(codes: torch.Tensor, scale: torch.Tensor) -> Optional[int]:
 
 
 def indexer_workspace(B: int, S: int, k: int, device) -> torch.Tensor:
-    return torch.empty(_lib.indexer_ws_bytes(B, S, k), dtype=torch.uint8, device=device)
+    return torch.empty(_lib.indexer_ws_bytes(int(B), int(S), int(k)), dtype=torch.uint8, device=device)
 
 
 def attention_workspace(B: int, H: int, D: int, n_comp: int, W: int, device) -> torch.Tensor:
-    return torch.empty(_lib.attention_ws_bytes(B, H, D, n_comp, W), dtype=torch.uint8, device=device)
+    n = _lib.attention_ws_bytes(int(B), int(H), int(D), int(n_comp), int(W))
+    return torch.empty(n, dtype=torch.uint8, device=device)
 
 
 def csa_indexer_topk_quant(index_q: torch.Tensor, index_weight: torch.Tensor, key_codes: torch.Tensor,
@@ -143,7 +144,7 @@ def csa_indexer_topk_quant(index_q: torch.Tensor, index_weight: torch.Tensor, ke
         _check_out("out", out, torch.int64, B * k, index_q.device)
     scores = torch.empty((B, k), dtype=torch.float32, device=index_q.device) if return_scores else None
     if workspace is None:
-        workspace = indexer_workspace(B, S, k, index_q.device)
+        workspace = torch.empty(_lib.indexer_ws_bytes(B, S, int(k)), dtype=torch.uint8, device=index_q.device)
     with torch.cuda.device(index_q.device):
         _lib.check(L.aekv_csa_indexer_topk_quant(
             _lib.ptr(q), _lib.ptr(w), _lib.ptr(codes), _lib.ptr(sc), _lib.ptr(diag), _lib.ptr(v), B, S, IH, IC, bits,
@@ -198,7 +199,7 @@ def quant_sink_attention(q: torch.Tensor, codes: torch.Tensor, scale: torch.Tens
     diag = quant._diag(D, q.device)
     n_comp = K if K >= 0 else S
     if workspace is None:
-        workspace = attention_workspace(B, H, D, n_comp, W, q.device)
+        workspace = torch.empty(_lib.attention_ws_bytes(B, H, D, n_comp, W), dtype=torch.uint8, device=q.device)
     dev = q.device
     if out is None:
         out = torch.empty(qs, dtype=torch.bfloat16, device=dev)
@@ -215,7 +216,8 @@ def quant_sink_attention(q: torch.Tensor, codes: torch.Tensor, scale: torch.Tens
 
 def decode_workspace(B: int, S: int, k: int, H: int, D: int, W: int, device) -> torch.Tensor:
     """Workspace of csa_decode_step (the indexer's and the attention's)."""
-    return torch.empty(_lib.decode_ws_bytes(B, S, k, H, D, W), dtype=torch.uint8, device=device)
+    n = _lib.decode_ws_bytes(int(B), int(S), int(k), int(H), int(D), int(W))
+    return torch.empty(n, dtype=torch.uint8, device=device)
 
 
 def csa_decode_step(q: torch.Tensor, index_q: torch.Tensor, index_weight: torch.Tensor, index_codes: torch.Tensor,
@@ -282,7 +284,7 @@ def csa_decode_step(q: torch.Tensor, index_q: torch.Tensor, index_weight: torch.
     else:
         _check_out("out", out, torch.bfloat16, B * H * D, dev)
     if workspace is None:
-        workspace = decode_workspace(B, S, k, H, D, W, dev)
+        workspace = torch.empty(_lib.decode_ws_bytes(B, S, int(k), H, D, W), dtype=torch.uint8, device=dev)
     with _lib.on_device(dev):
         rc = _lib.hot("aekv_csa_decode_quant")(
             iq.data_ptr(), iw.data_ptr(), ic.data_ptr(), isc.data_ptr(), idiag.data_ptr(), _iptr(v), B, S, IH, IC,

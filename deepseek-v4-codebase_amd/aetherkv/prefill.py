@@ -111,7 +111,7 @@ def csa_prefill_indexer_topk_quant(index_q: torch.Tensor, index_weight: torch.Te
         out = torch.empty((B, T, k), dtype=torch.int64, device=dev)
     scores = torch.empty((B, T, k), dtype=torch.float32, device=dev) if return_scores else None
     if workspace is None:
-        workspace = torch.empty(_lib.indexer_ws_bytes(B * T, S, k), dtype=torch.uint8, device=dev)
+        workspace = torch.empty(_lib.indexer_ws_bytes(B * T, S, int(k)), dtype=torch.uint8, device=dev)
     with _lib.on_device(dev):
         rc = _lib.hot("aekv_csa_prefill_indexer_topk_quant")(
             q.data_ptr(), w.data_ptr(), codes.data_ptr(), sc.data_ptr(), diag.data_ptr(), _iptr(v), B, T, S, IH, IC, bits,

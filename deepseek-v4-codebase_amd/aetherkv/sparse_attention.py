@@ -182,7 +182,7 @@ def _ext_csa_indexer_topk(index_q, index_kv, index_weight, k, mode="relu_w"):
         raise ValueError(f"mode must be one of {sorted(_lib.INDEX_MODES)}, got {mode!r}")
     dev = index_q.device
     out = torch.empty((B, k), dtype=torch.int64, device=dev)
-    ws = torch.empty(_lib.indexer_ws_bytes(B, S, k), dtype=torch.uint8, device=dev)
+    ws = torch.empty(_lib.indexer_ws_bytes(B, S, int(k)), dtype=torch.uint8, device=dev)
     with _lib.on_device(dev):
         rc = _lib.hot("aekv_csa_indexer_topk")(
             index_q.data_ptr(), index_kv.data_ptr(), index_weight.data_ptr(), None, B, S, IH, IC, int(k),

@@ -10,6 +10,7 @@ import torch
 
 import aetherkv._lib as L
 from aetherkv import sparse_sink_attention, tiled_prefill_attention
+from aetherkv.decode import attention_workspace, decode_workspace, indexer_workspace
 
 
 def test_captured_calls_get_buffers_of_their_own(monkeypatch):
@@ -67,3 +68,19 @@ def test_replays_after_a_larger_eager_call_on_the_capture_stream(dev, dtype, D):
             torch.cuda.synchronize()
             assert all(torch.equal(o, w) for o, w in zip(outs, want)), rep
             assert all(bool((t == float(i // 16)).all()) for i, t in enumerate(held)), rep
+
+
+def test_sizes_follow_a_tensor_count_changed_in_place():
+    # counts given as 0-d tensors: the size is that of the present value
+    k = torch.tensor(16)
+    small = indexer_workspace(4, 300, k, "cpu").numel()
+    k.fill_(2000)
+    assert indexer_workspace(4, 300, k, "cpu").numel() == L.lib().aekv_csa_indexer_workspace_size(4, 300, 2000) > small
+    n = torch.tensor(64)
+    small = decode_workspace(1, 300, 64, 12, 128, n, "cpu").numel()
+    n.fill_(4096)
+    assert decode_workspace(1, 300, 64, 12, 128, n, "cpu").numel() > small
+    n.fill_(64)
+    small = attention_workspace(1, 12, 128, n, 0, "cpu").numel()
+    n.fill_(4096)
+    assert attention_workspace(1, 12, 128, n, 0, "cpu").numel() > small
