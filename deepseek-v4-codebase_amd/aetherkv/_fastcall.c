@@ -36,6 +36,19 @@ static int want_args(Py_ssize_t nargs, Py_ssize_t n, const char* who) {
     const int rc_ = (call);                        \
     return PyLong_FromLong(rc_);                   \
   } while (0)
+/* The same with the interpreter lock released during the call, as ctypes does: a launch that waits (a
+ * full queue, the first load of a code object) does not stop the other Python threads.  The attention
+ * and decode-step calls keep the lock: two threads on one stream share a split workspace
+ * (aetherkv._lib.workspace, or the caller's own), and a call's kernels over it must be enqueued together. */
+#define RETURN_STATUS_UNLOCKED(call)               \
+  do {                                             \
+    int rc_;                                       \
+    if (PyErr_Occurred()) return NULL;             \
+    Py_BEGIN_ALLOW_THREADS                         \
+    rc_ = (call);                                  \
+    Py_END_ALLOW_THREADS                           \
+    return PyLong_FromLong(rc_);                   \
+  } while (0)
 
 /* aekv_sparse_sink_attention_ws(q, kv, idx, idx_dtype, sink, sink_numel, dtype, B, T, H, D, S, K,
  * scale, ws, ws_bytes, out, stream) */
@@ -150,7 +163,7 @@ static PyObject* f_tq_encode(PyObject* self, PyObject* const* args, Py_ssize_t n
   void* codes = ptr_arg(A(6));
   void* scale = ptr_arg(A(7));
   void* st = ptr_arg(A(8));
-  RETURN_STATUS(aekv_tq_encode(x, dt, n, d, bits, (const float*)diag, codes, (float*)scale, st));
+  RETURN_STATUS_UNLOCKED(aekv_tq_encode(x, dt, n, d, bits, (const float*)diag, codes, (float*)scale, st));
 }
 
 /* aekv_tq_decode(codes, scale, n_vec, d, bits, diag, out, out_dtype, stream) */
@@ -165,7 +178,7 @@ static PyObject* f_tq_decode(PyObject* self, PyObject* const* args, Py_ssize_t n
   void* out = ptr_arg(A(6));
   const int32_t odt = i32_arg(A(7));
   void* st = ptr_arg(A(8));
-  RETURN_STATUS(aekv_tq_decode(codes, (const float*)scale, n, d, bits, (const float*)diag, out, odt, st));
+  RETURN_STATUS_UNLOCKED(aekv_tq_decode(codes, (const float*)scale, n, d, bits, (const float*)diag, out, odt, st));
 }
 
 /* aekv_hca_compress(c, z, dtype, B, M, D, out, stream) */
@@ -178,7 +191,7 @@ static PyObject* f_hca_compress(PyObject* self, PyObject* const* args, Py_ssize_
   const int64_t B = i64_arg(A(3)), M = i64_arg(A(4)), D = i64_arg(A(5));
   void* out = ptr_arg(A(6));
   void* st = ptr_arg(A(7));
-  RETURN_STATUS(aekv_hca_compress(c, z, dt, B, M, D, out, st));
+  RETURN_STATUS_UNLOCKED(aekv_hca_compress(c, z, dt, B, M, D, out, st));
 }
 
 /* aekv_csa_indexer_topk(index_q, index_kv, index_weight, valid, B, S, IH, IC, k, mode, ws, ws_bytes, out_idx,
@@ -197,8 +210,9 @@ static PyObject* f_csa_indexer_topk(PyObject* self, PyObject* const* args, Py_ss
   void* oi = ptr_arg(A(12));
   void* os = ptr_arg(A(13));
   void* st = ptr_arg(A(14));
-  RETURN_STATUS(aekv_csa_indexer_topk((const float*)q, (const float*)kv, (const float*)w, (const int32_t*)valid, B, S, IH,
-                                      IC, k, mode, ws, wsb, (int64_t*)oi, (float*)os, st));
+  RETURN_STATUS_UNLOCKED(aekv_csa_indexer_topk((const float*)q, (const float*)kv, (const float*)w,
+                                               (const int32_t*)valid, B, S, IH, IC, k, mode, ws, wsb, (int64_t*)oi,
+                                               (float*)os, st));
 }
 
 /* aekv_csa_prefill_indexer_topk_quant(index_q, index_weight, key_codes, key_scale, diag, valid, B, T, S, IH, IC, bits, k,
@@ -219,9 +233,9 @@ static PyObject* f_csa_prefill_indexer(PyObject* self, PyObject* const* args, Py
   void* oi = ptr_arg(A(16));
   void* os = ptr_arg(A(17));
   void* st = ptr_arg(A(18));
-  RETURN_STATUS(aekv_csa_prefill_indexer_topk_quant((const float*)q, (const float*)w, kc, (const float*)ks,
-                                                    (const float*)diag, (const int32_t*)valid, B, T, S, IH, IC, bits, k,
-                                                    mode, ws, wsb, (int64_t*)oi, (float*)os, st));
+  RETURN_STATUS_UNLOCKED(aekv_csa_prefill_indexer_topk_quant(
+      (const float*)q, (const float*)w, kc, (const float*)ks, (const float*)diag, (const int32_t*)valid, B, T, S, IH, IC,
+      bits, k, mode, ws, wsb, (int64_t*)oi, (float*)os, st));
 }
 
 /* aekv_quant_prefill_attention(q, codes, scale, sel, visible, window, win_start, win_len, sink, diag, B, T, H, D, S,
@@ -239,9 +253,9 @@ static PyObject* f_quant_prefill_attention(PyObject* self, PyObject* const* args
   const size_t wsb = (size_t)i64_arg(A(20));
   void* out = ptr_arg(A(21));
   void* st = ptr_arg(A(22));
-  RETURN_STATUS(aekv_quant_prefill_attention(p[0], p[1], (const float*)p[2], (const int64_t*)p[3], (const int32_t*)p[4],
-                                             p[5], (const int32_t*)p[6], (const int32_t*)p[7], (const float*)p[8],
-                                             (const float*)p[9], B, T, H, D, S, ns, Wt, bits, sm, ws, wsb, out, st));
+  RETURN_STATUS_UNLOCKED(aekv_quant_prefill_attention(
+      p[0], p[1], (const float*)p[2], (const int64_t*)p[3], (const int32_t*)p[4], p[5], (const int32_t*)p[6],
+      (const int32_t*)p[7], (const float*)p[8], (const float*)p[9], B, T, H, D, S, ns, Wt, bits, sm, ws, wsb, out, st));
 }
 
 /* aekv_prefill_counts(B, T, start, n_blocks, compression, sliding_window, window_base, k, visible, selected, win_start,
@@ -256,8 +270,8 @@ static PyObject* f_prefill_counts(PyObject* self, PyObject* const* args, Py_ssiz
   void* ws = ptr_arg(A(10));
   void* wl = ptr_arg(A(11));
   void* st = ptr_arg(A(12));
-  RETURN_STATUS(aekv_prefill_counts(n[0], n[1], n[2], n[3], n[4], n[5], n[6], n[7], (int32_t*)vis, (int32_t*)sel,
-                                    (int32_t*)ws, (int32_t*)wl, st));
+  RETURN_STATUS_UNLOCKED(aekv_prefill_counts(n[0], n[1], n[2], n[3], n[4], n[5], n[6], n[7], (int32_t*)vis,
+                                             (int32_t*)sel, (int32_t*)ws, (int32_t*)wl, st));
 }
 
 static PyMethodDef methods[] = {
