@@ -39,6 +39,8 @@ int launch_f32_indexer(const float* q, const float* w, const float* keys, const 
                        int IH, int IC, int k, int mode, void* ws, int64_t* out_idx, float* out_score, hipStream_t st,
                        const char* who);
 bool use_specialised_codec();
+// HIP refuses a launch of more work-items than this in one grid dimension.
+constexpr int64_t kMaxGridThreads = 0xffffffffLL;
 // Host-side argument checks of the quantised-key indexer for B * T rows (csa_indexer.hip).
 int validate_quant_rows(const float* index_q, const float* index_weight, const void* key_codes,
                         const float* key_scale, const float* diag, int64_t B, int64_t T, int64_t S, int32_t IH,

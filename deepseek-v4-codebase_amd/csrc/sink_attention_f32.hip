@@ -404,7 +404,14 @@ bool sink_attention_f32_supported(int32_t dtype, int64_t D) {
 
 bool sink_attention_f32_fits(bool dense, int64_t D, int64_t B, int64_t T, int64_t H, int64_t S, int64_t K) {
   const int64_t lim = 0x7fffffff - 4096;  // (32-bit positions, a few groups past the end among them)
-  return S <= lim && K <= lim && B * T * H <= lim && T * H <= lim && f32_plan(dense, D, B, T, H, K, false).wgs <= lim;
+  if (S > lim || K > lim || B * T * H > lim || T * H > lim) return false;
+  // (256 or 512 threads per 16 or 32 rows, where the VALU kernel takes 64 per row: sparse calls of many
+  // targets with few heads reach the launch's limit first here)
+  for (const bool split : {false, true}) {
+    const F32Plan p = f32_plan(dense, D, B, T, H, K, split);
+    if (p.wgs * 64 * p.nw > kMaxGridThreads) return false;
+  }
+  return true;
 }
 
 size_t sink_attention_f32_workspace(bool dense, int64_t D, int64_t B, int64_t T, int64_t H, int64_t K) {

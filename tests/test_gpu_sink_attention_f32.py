@@ -103,3 +103,20 @@ def test_no_sink_and_no_maximum(dev, K):
     idx[0, 0] = -1
     got = sparse_sink_attention(q.to(dev), kv.to(dev), idx.to(dev), torch.full((12,), float("-inf"), device=dev), 128 ** -0.5)
     assert bool((got[0, 0] == 0).all()) and bool(torch.isnan(got[0, 1]).all())
+
+
+def test_more_targets_than_a_launch_of_whole_workgroups(dev):
+    # 2^24 targets of one head: a workgroup of 256 threads each would be 2^32 work-items, past what a
+    # launch takes, so the call runs on the kernel of one wave per row; its parts fit
+    T, D, S = 1 << 24, 64, 512
+    g = torch.Generator(device=dev).manual_seed(3)
+    q = torch.randn(1, T, 1, D, generator=g, device=dev, dtype=torch.bfloat16)
+    kv = torch.randn(1, S, 2, D, generator=g, device=dev, dtype=torch.bfloat16)
+    idx = torch.randint(0, S, (1, T, 2), generator=g, device=dev, dtype=torch.int32)
+    sink = torch.zeros(1, device=dev, dtype=torch.bfloat16)
+    got = sparse_sink_attention(q, kv, idx, sink, D ** -0.5)
+    for lo in (0, T // 2, T - 4096):
+        part = slice(lo, lo + 4096)
+        want = sparse_sink_attention(q[:, part].contiguous(), kv, idx[:, part].contiguous(), sink, D ** -0.5)
+        # both in fp32 from the same inputs: at most one bf16 rounding apart
+        torch.testing.assert_close(got[:, part], want, rtol=2 ** -7, atol=1e-5)
