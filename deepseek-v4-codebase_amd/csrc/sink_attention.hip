@@ -417,17 +417,19 @@ __global__ __launch_bounds__(kThreads) void hca_compress_rows_kernel(const uint4
 }
 
 // Launches the kernel above when the row's entries fit (at most 4 entries per lane of a wave, else at
-// most 16 per lane of a workgroup); false: nothing launched.
+// most 16 per lane of a workgroup) and the rows' threads fit one launch (the general kernel takes a
+// thread per column, fewer where rows are narrower than the team); false: nothing launched.
 template <int DT>
 bool launch_compress_rows(const void* c, const void* z, int64_t B, int64_t M, int64_t D, void* out, hipStream_t st) {
   const int64_t ncol = D * static_cast<int64_t>(dtype_size(DT)) / 16;
   if (ncol < 1 || ncol > 64 || !is_pow2(ncol) || D * static_cast<int64_t>(dtype_size(DT)) % 16 != 0 ||
-      !is_aligned(c, 16) || !is_aligned(z, 16) || B > 0x7fffffffLL)
+      !is_aligned(c, 16) || !is_aligned(z, 16))
     return false;
   const int64_t wave_groups = 64 / ncol, wg_groups = 256 / ncol;
   const uint4* cv = static_cast<const uint4*>(c);
   const uint4* zv = static_cast<const uint4*>(z);
   auto go = [&](auto fn, int64_t grid) {
+    if (grid > kMaxGridThreads / kThreads) return false;
     hipLaunchKernelGGL(fn, dim3(static_cast<uint32_t>(grid)), dim3(kThreads), 0, st, cv, zv, B, static_cast<int>(M),
                        static_cast<int>(ncol), out);
     return true;

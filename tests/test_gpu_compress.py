@@ -44,3 +44,13 @@ def test_infinities_stay_in_their_column(dev):
     view.copy_(z)
     torch.testing.assert_close(hca_compress(view, z.to(dev)), hca_compress(z.to(dev), z.to(dev)), rtol=1e-5, atol=1e-5,
                                equal_nan=True)
+
+
+def test_more_rows_than_a_launch_of_whole_waves(dev):
+    # 2^26 rows of 16 bytes: a wave each would be 2^32 work-items, past what a launch takes, so the call
+    # runs on the general kernel (one entry per row: the result is the row itself)
+    B, D = 1 << 26, 8
+    c = torch.randint(-100, 100, (B, 1, D), device=dev, dtype=torch.int8).to(torch.bfloat16)
+    z = torch.zeros_like(c)
+    got = hca_compress(c, z)
+    assert torch.equal(got, c[:, 0])
