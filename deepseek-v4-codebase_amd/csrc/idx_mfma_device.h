@@ -1068,27 +1068,10 @@ __device__ __forceinline__ uint32_t select_row(const MfmaIdxArgs& a, const int b
 
   // ---- 2. three radix levels down to the kk-th largest key T ----
   // Passes over all of the row's stored keys (candidates that overflow LDS), four adjacent keys per
-  // lane: vector v holds keys 4 v .. 4 v + 3 (those at or past the count are not the row's).  f(key,
-  // index, in) is called by whole waves.
+  // lane: vector v holds keys 4 v .. 4 v + 3 (those at or past the count are not the row's).
   const int nv_i = static_cast<int>(nv), n_vec = (nv_i + 3) >> 2;
   auto load_vec = [&](int v) {
     return static_cast<u32x4_t>(__builtin_amdgcn_raw_buffer_load_b128(krs, static_cast<uint32_t>(v) * 16u, 0, 0));
-  };
-  auto for_part_keys = [&](int v0, int v1, auto&& f) {  // this wave alone
-#pragma unroll 1
-    for (int v = v0; v < v1; v += 64) {
-      const u32x4_t kw = load_vec(v + lane);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) f(kw[e], 4 * (v + lane) + e, 4 * (v + lane) + e < nv_i && v + lane < v1);
-    }
-  };
-  auto for_all_keys = [&](int v0, int v1, auto&& f) {  // every wave its share of the workgroup's steps
-#pragma unroll 1
-    for (int v = v0 + 64 * wv; v < v1; v += NT) {
-      const u32x4_t kw = load_vec(v + lane);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) f(kw[e], 4 * (v + lane) + e, 4 * (v + lane) + e < nv_i);
-    }
   };
   uint32_t need = kk;  // keys still to take at or below the current prefix
   uint32_t prefix = 0u;
@@ -1109,19 +1092,44 @@ __device__ __forceinline__ uint32_t select_row(const MfmaIdxArgs& a, const int b
         if (lvl == 0 || (key >> shift) == prefix) atomicAdd(&h[(key >> nshift) & mask], 1u);
       }
     } else {
-      // Rows come here because many keys are equal, so lanes of a wave mostly meet in one bin: the
-      // bin of the wave's first counted key takes one atomic for all of its lanes there.
-      for_all_keys(0, n_vec, [&](const uint32_t key, const int, const bool in) {
-        const bool act = in && (lvl == 0 || (key >> shift) == prefix);
-        const uint64_t am = __builtin_amdgcn_ballot_w64(act);
-        if (am == 0u) return;  // wave-uniform
-        const uint32_t bin = (key >> nshift) & mask;
-        const int first = __builtin_ctzll(am);
-        const uint32_t b0 = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(bin), first));
-        const uint64_t same = __builtin_amdgcn_ballot_w64(act && bin == b0);
-        if (lane == first) atomicAdd(&h[b0], static_cast<uint32_t>(__builtin_popcountll(same)));
-        if (act && bin != b0) atomicAdd(&h[bin], 1u);
-      });
+      // Rows come here because many keys are equal, or because they have fewer slots than k and too
+      // many keys for the candidates' LDS (NT = 512: 1537 to 16 k keys).  Where a quarter of a wave's
+      // first keys meet in one bin, the bin of each element's first counted key takes one atomic for all
+      // of its lanes there; elsewhere each key takes its own (aggregated throughout, a row of 3000
+      // distinct keys took 1 us longer).
+#pragma unroll 1
+      for (int v = 64 * wv; v < n_vec; v += NT) {
+        const u32x4_t kw = load_vec(v + lane);
+        bool act[4];
+        uint32_t bin[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          act[e] = 4 * (v + lane) + e < nv_i && (lvl == 0 || (kw[e] >> shift) == prefix);
+          bin[e] = (kw[e] >> nshift) & mask;
+        }
+        auto first_bin = [&](int e, uint64_t am) {  // bin of the first lane of am
+          return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(bin[e]), __builtin_ctzll(am)));
+        };
+        const uint64_t am0 = __builtin_amdgcn_ballot_w64(act[0]);
+        bool meet = false;  // wave-uniform
+        if (am0 != 0u) {
+          const uint32_t b0 = first_bin(0, am0);
+          meet = __builtin_popcountll(__builtin_amdgcn_ballot_w64(act[0] && bin[0] == b0)) >= 16;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (!meet) {
+            if (act[e]) atomicAdd(&h[bin[e]], 1u);
+            continue;
+          }
+          const uint64_t am = __builtin_amdgcn_ballot_w64(act[e]);
+          if (am == 0u) continue;  // wave-uniform
+          const uint32_t b0 = first_bin(e, am);
+          const uint64_t same = __builtin_amdgcn_ballot_w64(act[e] && bin[e] == b0);
+          if (lane == __builtin_ctzll(am)) atomicAdd(&h[b0], static_cast<uint32_t>(__builtin_popcountll(same)));
+          if (act[e] && bin[e] != b0) atomicAdd(&h[bin[e]], 1u);
+        }
+      }
     }
     __syncthreads();
     uint32_t t, ab, ct;
@@ -1167,13 +1175,28 @@ __device__ __forceinline__ uint32_t select_row(const MfmaIdxArgs& a, const int b
     const int per = (n_vec + NW * 64 - 1) / (NW * 64) * 64;  // whole wave steps
     const int v0 = wv * per, v1 = min(n_vec, v0 + per);
     uint32_t eq = 0u;  // wave-uniform
-    for_part_keys(v0, v1, [&](const uint32_t key, const int j, const bool in) {
-      const bool gt = in && key > T;
-      eq += static_cast<uint32_t>(__builtin_popcountll(__builtin_amdgcn_ballot_w64(in && key == T)));
-      if (__builtin_amdgcn_ballot_w64(gt) == 0u) return;  // wave-uniform
-      const uint32_t pg = wave_reserve<1>(&s_cnt[0], gt ? 1u : 0u);
-      if (gt && pg < n_gt) sel[pg] = sort_word(key, static_cast<uint32_t>(j));
-    });
+#pragma unroll 1
+    for (int v = v0; v < v1; v += 64) {
+      const u32x4_t kw = load_vec(v + lane);
+      uint32_t gt4 = 0u, eq_lane = 0u;  // bit e: key e > T; the lane's keys == T
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool in = 4 * (v + lane) + e < nv_i;
+        gt4 |= in && kw[e] > T ? 1u << e : 0u;
+        eq_lane += in && kw[e] == T ? 1u : 0u;
+      }
+#pragma unroll
+      for (int bit = 0; bit < 3; ++bit)
+        eq += static_cast<uint32_t>(__builtin_popcountll(__builtin_amdgcn_ballot_w64(((eq_lane >> bit) & 1u) != 0u))) << bit;
+      if (__builtin_amdgcn_ballot_w64(gt4 != 0u) == 0u) continue;  // wave-uniform
+      uint32_t pg = wave_reserve<3>(&s_cnt[0], static_cast<uint32_t>(__builtin_popcount(gt4)));
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if ((gt4 >> e) & 1u) {
+          if (pg < n_gt) sel[pg] = sort_word(kw[e], static_cast<uint32_t>(4 * (v + lane) + e));
+          ++pg;
+        }
+    }
     if (lane == 0) s_wave_eq[wv] = eq;
     __syncthreads();
     uint32_t run = 0u;  // keys == T before the current step
@@ -1183,7 +1206,7 @@ __device__ __forceinline__ uint32_t select_row(const MfmaIdxArgs& a, const int b
       const u32x4_t kw = load_vec(v + lane);
       uint32_t m4 = 0u;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) m4 |= (4 * (v + lane) + e < nv_i && v + lane < v1 && kw[e] == T) ? (1u << e) : 0u;
+      for (int e = 0; e < 4; ++e) m4 |= (4 * (v + lane) + e < nv_i && kw[e] == T) ? (1u << e) : 0u;
       const uint32_t cnt = static_cast<uint32_t>(__builtin_popcount(m4));
       uint32_t pos = run, tot = 0u;
 #pragma unroll

@@ -110,3 +110,23 @@ def test_many_equal_scores(dev, S, k, top):
     idx = csa_indexer_topk(q.to(dev), kv.to(dev), w.to(dev), k, mode="raw").cpu()
     want = (top + [j for j in range(k + len(top)) if j not in top])[:k]
     assert idx.tolist() == [want, want]
+
+
+# Rows with fewer 16-key slots than k and more keys than a workgroup collects: every stored key is counted.
+# Whole-number scores, so that the selection is exact: mostly distinct ones, a few hundred values, and a few
+# values (where whole waves meet in one bin).  1024 rows take the 512-thread select (1536 candidates), 2 rows
+# the 1024-thread one (4096).
+@pytest.mark.parametrize("B,S,k", [(1024, 1537, 256), (1024, 2049, 129), (1024, 3001, 200), (1024, 2047, 512),
+                                   (2, 4097, 1024), (2, 8190, 513), (2, 16383, 1024)])
+@pytest.mark.parametrize("values", [1 << 20, 300, 3])
+def test_fewer_slots_than_k(dev, B, S, k, values):
+    g = torch.Generator(device=dev).manual_seed(S + values)
+    s = torch.randint(-values // 8, values, (B, S), generator=g, device=dev).float()
+    s[0] = s[0].sort().values  # (ordered along the row: whole waves above or below the k-th key)
+    kv = torch.zeros(B, S, 64, device=dev)
+    kv[:, :, 5] = s
+    q = torch.zeros(B, 1, 64, device=dev)
+    q[:, :, 5] = 1.0
+    idx = csa_indexer_topk(q, kv, torch.ones(B, 1, device=dev), k, mode="relu_w")
+    want = s.sort(dim=1, descending=True, stable=True).indices[:, :k]
+    assert torch.equal(idx, want)
