@@ -51,14 +51,11 @@ bool quant_attn_mfma_supported(int64_t H, int64_t D);
 bool quant_attn_mfma_fits(int64_t rows, int64_t n_src);  // grid and split-combine limits
 // Chunked-prefill HCA attention over bf16 blocks [B, S, 128] already decoded (prefill_flash.hip).
 bool hca_prefill_flash_supported(int64_t H, int64_t D);
-// The workspace: the decoded blocks (hca_prefill_flash_blocks bytes), then the results of the row blocks that
-// are split; without room for those (part null or too small) no block is split.
-size_t hca_prefill_flash_blocks(int64_t B, int64_t S);
-size_t hca_prefill_flash_workspace(int64_t B, int64_t T, int64_t H, int64_t S);
+size_t hca_prefill_flash_workspace(int64_t B, int64_t S);  // the decoded blocks
 int launch_hca_prefill_flash(const void* q, const void* kblk, const void* window, const int32_t* vis,
                              const int32_t* wstart, const int32_t* wlen, const float* sink, int64_t B, int64_t T,
-                             int64_t H, int64_t S, int64_t Wt, float softmax_scale, void* part, size_t part_bytes,
-                             void* out, hipStream_t st, const char* who);
+                             int64_t H, int64_t S, int64_t Wt, float softmax_scale, void* out, hipStream_t st,
+                             const char* who);
 // Drop-in sink attention on the matrix cores, head_dim 128, bf16/fp16 (sink_attention_mfma.hip):
 // q [B, T, H, 128], kv [B, S, 2, 128], per-target indices idx [B, T, K] (idx_kind 4/8: int32/int64)
 // or every source (idx_kind 0, K = S).  A workspace (may be null) lets launches with few

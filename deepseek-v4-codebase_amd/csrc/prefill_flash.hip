@@ -49,10 +49,8 @@
 // the very bf16 weights the numerator used: each lane adds its own weights of the row with
 // v_dot2_f32_bf16 (f16) against ones, and the two lane halves are added at the end.  Tiles that
 // every row of the workgroup sees in full skip the masks.
-#include <algorithm>
 #include <atomic>
 
-#include "sink_combine.h"
 #include "tq_device.h"
 
 namespace aekv {
@@ -94,7 +92,7 @@ struct FlashGeom {
   static constexpr int kPass = 1024 * kLoadWaves;       // bytes of a tile per staging pass
   static constexpr int kChunks = kTileBytes / kPass;    // staging passes per tile
   static constexpr int kVOff = ROWB == 256 ? 0 : 256;   // V's byte offset in a row
-  static constexpr bool kDense = ROWB == 512;           // every source, no counts
+  static constexpr bool kSplit = ROWB == 512;           // the dense caller may split a row's sources
   static constexpr int kSlots = RG * KS / 2;            // merge states in LDS at once (16 KB each)
   static constexpr int kMergeExtra = kSlots > 4 ? (kSlots - 4) * kSlotFloats * 4 : 16;  // beyond the tiles
   static_assert(kKB >= 1 && kKW % 32 == 0, "tiles are whole 32-key blocks per wave");
@@ -175,12 +173,8 @@ struct FlashArgs {
   uint32_t gx;            // workgroups per sequence
   int H;
   float scale2;           // softmax scale * log2(e)
-  // The first n_full row blocks (of all sequences, in order) run whole, a workgroup each; the others in
-  // n_split pieces of their source tiles, a workgroup each, whose results go to part.
-  uint32_t n_full;
-  int n_split;
-  float* part;            // [row, n_split, 132]: max, sum (log2 units), 2 pad, O[128]; row = (b, t, h)
-                          // (dense) or 32 RG (block - n_full) + row of the block (HCA)
+  int n_split;            // source pieces per row block (1: the workgroup finishes its rows)
+  float* part;            // [B * T * H, n_split, 132]: max, sum (log2 units), 2 pad, O[128]
   uint16_t* out;          // [B, T, H, 128]
 };
 
@@ -188,9 +182,7 @@ struct FlashArgs {
 // loop (the matrix instructions take VGPR operands) instead of moving to AGPRs and back, and the
 // scheduler may spend registers on reading LDS operands ahead of the products.  A launch has about
 // 1.5 workgroups per CU at the bench shape, so more resident waves would not exist anyway.
-// SPLIT: some row blocks run in pieces of their source tiles (FlashArgs::n_full); without, the kernel has no
-// trace of them (1 us of 42 with the piece bounds carried through whole blocks).
-template <int DT, int ROWB, int RG, int KS, bool SPLIT>
+template <int DT, int ROWB, int RG, int KS>
 __global__ __launch_bounds__(64 * RG * KS) __attribute__((
     amdgpu_waves_per_eu(FlashGeom<ROWB, RG, KS>::kWavesPerSimd, FlashGeom<ROWB, RG, KS>::kWavesPerSimd))) void
 flash_sink_attn_kernel(FlashArgs a) {
@@ -211,21 +203,14 @@ flash_sink_attn_kernel(FlashArgs a) {
   // that XCD x runs the consecutive range [x n/8, (x+1) n/8), i.e. whole sequences, whose blocks
   // then stay in that XCD's L2 instead of every L2 streaming every sequence.
   // (32-bit index arithmetic: the launcher bounds the grid and B * T * H below 2^31)
-  // (The whole blocks and the pieces are renumbered each within their own range.)
-  auto xcd_order = [](uint32_t i, uint32_t n) { return n % 8 == 0 ? (i % 8) * (n / 8) + i / 8 : i; };
-  uint32_t blk, nsp = 1u;
-  int split = 0;
-  const uint32_t n_full = SPLIT ? a.n_full : gridDim.x;
-  if (!SPLIT || blockIdx.x < n_full) {  // workgroup-uniform
-    blk = xcd_order(blockIdx.x, n_full);
-  } else {
-    const uint32_t i = xcd_order(blockIdx.x - n_full, n_full % 8 == 0 ? gridDim.x - n_full : 1u);
-    nsp = static_cast<uint32_t>(a.n_split);
-    blk = n_full + i / nsp;
-    split = static_cast<int>(i % nsp);
-  }
-  const int b = static_cast<int>(blk / a.gx);
-  const int wrow = static_cast<int>(blk % a.gx);
+  const uint32_t n_wg = gridDim.x;
+  uint32_t wgi = blockIdx.x;
+  if (n_wg % 8 == 0) wgi = (wgi % 8) * (n_wg / 8) + wgi / 8;
+  const uint32_t nsp = Gm::kSplit ? static_cast<uint32_t>(a.n_split) : 1u;
+  const uint32_t per_seq = a.gx * nsp;
+  const int b = static_cast<int>(wgi / per_seq);
+  const int wrow = static_cast<int>((wgi % per_seq) / nsp);
+  const int split = static_cast<int>(wgi % nsp);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (a scalar register)
   const int rh = wv % RG, kh = wv / RG;  // row group, key split
@@ -286,8 +271,8 @@ flash_sink_attn_kernel(FlashArgs a) {
   const int n_wt = whi > wlo ? (whi - wlo + kFTile - 1) / kFTile : 0;
   const int n_tiles = n_bt + n_wt;
   // this workgroup's tiles [it0, it1): one piece of n_split
-  const int tps = SPLIT ? (n_tiles + static_cast<int>(nsp) - 1) / static_cast<int>(nsp) : n_tiles;
-  const int it0 = SPLIT ? min(split * tps, n_tiles) : 0, it1 = SPLIT ? min(it0 + tps, n_tiles) : n_tiles;
+  const int tps = (n_tiles + static_cast<int>(nsp) - 1) / static_cast<int>(nsp);
+  const int it0 = min(split * tps, n_tiles), it1 = min(it0 + tps, n_tiles);
 
   // the row's query as the B operand of S^T = K Q^T: dims 16 ks + 8 hh .. + 7
   v8 qb[8];
@@ -503,11 +488,9 @@ flash_sink_attn_kernel(FlashArgs a) {
     }
   }
   if (kh != 0 || !rv) return;
-  if (SPLIT && nsp > 1) {
+  if (Gm::kSplit && nsp > 1) {
     // one piece: the row's (max, sum, O) relative to its max, merged with the sink by the combine
-    const int64_t prow = Gm::kDense ? static_cast<int64_t>(b) * RT + r
-                                    : static_cast<int64_t>(blk - n_full) * Gm::kRows + (32 * rh + rl);
-    float* dst = a.part + (prow * nsp + split) * (kFD + 4);
+    float* dst = a.part + ((static_cast<int64_t>(b) * RT + r) * a.n_split + split) * (kFD + 4);
     if (hh == 0) {
       dst[0] = m_run;
       dst[1] = lsum;
@@ -543,6 +526,10 @@ flash_sink_attn_kernel(FlashArgs a) {
 }
 
 }  // namespace
+
+size_t hca_prefill_flash_workspace(int64_t B, int64_t S) {
+  return align_up(static_cast<size_t>(B) * static_cast<size_t>(S) * kFD * 2, 256);
+}
 
 bool hca_prefill_flash_supported(int64_t H, int64_t D) { return D == kFD && H >= 1; }
 
@@ -588,71 +575,24 @@ int64_t device_cus() {
 
 }  // namespace
 
-namespace {
-
-// How an HCA launch is divided.  The shape with the shorter schedule is taken: 43 us per round of 256 wide
-// workgroups; 50 us per round of 512 narrow ones, and for a last round of at most 256 (one per CU) 33 us, or
-// 19 us after a full one (12 heads x 2048 blocks; narrow / wide: 1360 targets 33 / 40 us, 2048 47 / 43,
-// 2400 48 / 76, 3001 69 / 78).  Narrow blocks of a last round of at most 128 are split into as many pieces
-// of their source tiles as give every CU a workgroup (at least 4 tiles each).  Measured, kernel and combine:
-// 128 targets 13.6 + 4 us (29 unsplit), 340 targets 16.9 + 4 (29), 3001 targets 54.5 + 4.7 (69).
-struct HcaPlan {
-  bool wide;
-  int64_t n_full, n_rest;  // row blocks run whole, and split
-  int n_split;
-  size_t part;             // bytes of the pieces' results
-};
-
-HcaPlan hca_plan(int64_t B, int64_t T, int64_t H, int64_t S, bool may_split) {
+// The 96-row shape when it leaves fewer rows on the busiest CU: two 64-row workgroups or one
+// 96-row workgroup per CU at a time (e.g. 8 x 3072 rows: 384 narrow workgroups put 128 rows on
+// half of the 256 CUs; 256 wide ones put 96 on each).
+bool hca_flash_wide(int64_t B, int64_t T, int64_t H) {
   const int forced = g_hca_rows.load(std::memory_order_relaxed);
+  if (forced) return forced == HcaWide::kRows;
   const int64_t cus = device_cus();
-  const int64_t n_wide = B * ceil_div(T * H, int64_t(HcaWide::kRows)), n = B * ceil_div(T * H, int64_t(HcaNarrow::kRows));
-  const int64_t full = n / (2 * cus), rem = n % (2 * cus);
-  const int64_t narrow_us = 50 * full + (rem == 0 ? 0 : rem > cus ? 50 : full > 0 ? 19 : 33);
-  HcaPlan p{};
-  p.n_split = 1;
-  p.wide = forced ? forced == HcaWide::kRows : 43 * ceil_div(n_wide, cus) < narrow_us;
-  p.n_full = p.wide ? n_wide : n;
-  const int64_t tiles = ceil_div(S, int64_t(HcaNarrow::kTile)) + 2;
-  if (!p.wide && may_split && rem > 0 && rem <= cus / 2 && tiles >= 8) {
-    p.n_split = static_cast<int>(std::min<int64_t>(std::min(cus / rem, tiles / 4), 8));
-    p.n_full = n - rem;
-    p.n_rest = rem;
-    p.part = align_up(static_cast<size_t>(rem * HcaNarrow::kRows * p.n_split) * (kFD + 4) * sizeof(float), 256);
-  }
-  return p;
-}
-
-// Row `i` of the split blocks' rows -> (b, t, h) row and sink head of the combine; -1: past the sequence.
-struct BlockRows {
-  uint32_t first, gx, block_rows, seq_rows;  // first split block, blocks per sequence, rows of each
-  __device__ int64_t operator()(uint32_t i, int& head, int H) const {
-    const uint32_t blk = first + i / block_rows;
-    const uint32_t b = blk / gx, r = (blk - b * gx) * block_rows + i % block_rows;
-    head = static_cast<int>(r % static_cast<uint32_t>(H));
-    return r < seq_rows ? static_cast<int64_t>(b) * seq_rows + r : -1;
-  }
-};
-
-}  // namespace
-
-// The decoded blocks, then the pieces' results.
-size_t hca_prefill_flash_blocks(int64_t B, int64_t S) {
-  return align_up(static_cast<size_t>(B) * static_cast<size_t>(S) * kFD * 2, 256);
-}
-
-size_t hca_prefill_flash_workspace(int64_t B, int64_t T, int64_t H, int64_t S) {
-  return hca_prefill_flash_blocks(B, S) + hca_plan(B, T, H, S, true).part;
+  const int64_t n_narrow = B * ceil_div(T * H, HcaNarrow::kRows), n_wide = B * ceil_div(T * H, HcaWide::kRows);
+  return ceil_div(n_wide, cus) * HcaWide::kRows < ceil_div(n_narrow, 2 * cus) * 2 * HcaNarrow::kRows;
 }
 
 int launch_hca_prefill_flash(const void* q, const void* kblk, const void* window, const int32_t* vis,
                              const int32_t* wstart, const int32_t* wlen, const float* sink, int64_t B, int64_t T,
-                             int64_t H, int64_t S, int64_t Wt, float softmax_scale, void* part, size_t part_bytes,
-                             void* out, hipStream_t st, const char* who) {
+                             int64_t H, int64_t S, int64_t Wt, float softmax_scale, void* out, hipStream_t st,
+                             const char* who) {
   FlashArgs a{};
-  HcaPlan p = hca_plan(B, T, H, S, part != nullptr);
-  if (p.part > part_bytes) p = hca_plan(B, T, H, S, false);  // (the split is only a faster schedule)
-  const int rows = p.wide ? HcaWide::kRows : HcaNarrow::kRows;
+  const bool wide = hca_flash_wide(B, T, H);
+  const int rows = wide ? HcaWide::kRows : HcaNarrow::kRows;
   if (int rc = flash_prepare(a, B, T, H, S, Wt, HcaNarrow::kTile, rows, softmax_scale, who)) return rc;
   if (T * H == 0 || B == 0) return AEKV_OK;
   a.q = static_cast<const uint16_t*>(q);
@@ -664,19 +604,11 @@ int launch_hca_prefill_flash(const void* q, const void* kblk, const void* window
   a.sink = sink;
   a.sink_dt = AEKV_F32;
   a.sink_scalar = 0;
-  a.n_full = static_cast<uint32_t>(p.n_full);
-  a.n_split = p.n_split;
-  a.part = static_cast<float*>(part);
+  a.n_split = 1;
   a.out = static_cast<uint16_t*>(out);
-  const dim3 grid(static_cast<uint32_t>(p.n_full + p.n_rest * p.n_split));
-  auto fn = p.wide         ? flash_sink_attn_kernel<AEKV_BF16, 256, 3, 4, false>
-            : p.n_rest > 0 ? flash_sink_attn_kernel<AEKV_BF16, 256, 2, 2, true>
-                           : flash_sink_attn_kernel<AEKV_BF16, 256, 2, 2, false>;
-  hipLaunchKernelGGL(fn, grid, dim3(p.wide ? HcaWide::kThreads : HcaNarrow::kThreads), 0, st, a);
-  if (int rc = check_launch(who)) return rc;
-  if (p.n_rest == 0) return AEKV_OK;
-  const BlockRows map{static_cast<uint32_t>(p.n_full), a.gx, static_cast<uint32_t>(rows), static_cast<uint32_t>(T * H)};
-  sinkc::launch_combine<AEKV_BF16, kFD, AEKV_F32>(a.part, p.n_split, sink, 0, a.H, p.n_rest * rows, out, st, map);
+  const dim3 grid(a.gx * static_cast<uint32_t>(B));
+  if (wide) hipLaunchKernelGGL((flash_sink_attn_kernel<AEKV_BF16, 256, 3, 4>), grid, dim3(HcaWide::kThreads), 0, st, a);
+  else hipLaunchKernelGGL((flash_sink_attn_kernel<AEKV_BF16, 256, 2, 2>), grid, dim3(HcaNarrow::kThreads), 0, st, a);
   return check_launch(who);
 }
 
@@ -691,7 +623,6 @@ int launch_dense_flash_attention(const void* q, const void* kv, const void* sink
   if (T * H == 0 || B == 0) return AEKV_OK;
   if (n_split < 1 || (n_split > 1 && !part)) return fail(AEKV_ERR_VALUE, "%s: bad source split", who);
   if (static_cast<int64_t>(a.gx) * B * n_split > 0x7fffffff) return fail(AEKV_ERR_UNSUPPORTED, "%s: grid too large", who);
-  a.n_full = 0;
   a.n_split = n_split;
   a.part = part;
   a.q = static_cast<const uint16_t*>(q);
@@ -702,8 +633,8 @@ int launch_dense_flash_attention(const void* q, const void* kv, const void* sink
   a.out = static_cast<uint16_t*>(out);
   const dim3 grid(a.gx * static_cast<uint32_t>(B) * static_cast<uint32_t>(n_split));
   if (dtype == AEKV_F16)
-    hipLaunchKernelGGL((flash_sink_attn_kernel<AEKV_F16, 512, 2, 2, true>), grid, dim3(DenseGeom::kThreads), 0, st, a);
-  else hipLaunchKernelGGL((flash_sink_attn_kernel<AEKV_BF16, 512, 2, 2, true>), grid, dim3(DenseGeom::kThreads), 0, st, a);
+    hipLaunchKernelGGL((flash_sink_attn_kernel<AEKV_F16, 512, 2, 2>), grid, dim3(DenseGeom::kThreads), 0, st, a);
+  else hipLaunchKernelGGL((flash_sink_attn_kernel<AEKV_BF16, 512, 2, 2>), grid, dim3(DenseGeom::kThreads), 0, st, a);
   return check_launch(who);
 }
 

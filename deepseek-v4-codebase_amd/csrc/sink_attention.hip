@@ -665,9 +665,9 @@ extern "C" int aekv_quant_sink_attention(const void* q, const void* codes, const
 extern "C" size_t aekv_quant_prefill_workspace_size(int64_t B, int64_t T, int64_t H, int64_t n_comp, int64_t Wt) {
   if (B <= 0 || T <= 0 || H <= 0) return 256;
   const int64_t nc = std::max<int64_t>(n_comp, 0);
-  // per-target split partials (CSA), or every block decoded to bf16 and the split row blocks (HCA: n_comp = S)
+  // per-target split partials (CSA) or every block decoded to bf16 (HCA: n_comp = S)
   const size_t rows = quant_attn_mfma_workspace(B * T, H, nc + std::max<int64_t>(Wt, 0));
-  const size_t blocks = hca_prefill_flash_workspace(B, T, H, nc);
+  const size_t blocks = hca_prefill_flash_workspace(B, nc);
   return std::max<size_t>(256, std::max(rows, blocks));
 }
 
@@ -699,17 +699,15 @@ extern "C" int aekv_quant_prefill_attention(const void* q, const void* codes, co
   if (all_blocks && hca_prefill_flash_supported(H, D)) {
     // HCA: decode every block once (exactly PolarQuant.decode's bf16 values) into the workspace,
     // then the flash kernel over [blocks; window] with per-target masks
-    const size_t need = S > 0 ? hca_prefill_flash_blocks(B, S) : 0;
+    const size_t need = S > 0 ? hca_prefill_flash_workspace(B, S) : 0;
     if (need > 0 && (!ws || ws_bytes < need))
       return fail(AEKV_ERR_WORKSPACE, "%s: workspace of %zu bytes required, got %zu", who, need, ws_bytes);
     if (need > 0 && !is_aligned(ws, 256)) return fail(AEKV_ERR_ALIGN, "%s: workspace must be 256-byte aligned", who);
     if (S > 0) {
       if (int rc = aekv_tq_decode(codes, scale, B * S, 128, bits, diag, ws, AEKV_BF16, stream)) return rc;
     }
-    const bool room = need > 0 && ws_bytes > need;
-    return launch_hca_prefill_flash(q, ws, window, visible, win_start, win_len, sink, B, T, H, S, Wt, softmax_scale,
-                                    room ? static_cast<char*>(ws) + need : nullptr, room ? ws_bytes - need : 0, out,
-                                    as_stream(stream), who);
+    return launch_hca_prefill_flash(q, ws, window, visible, win_start, win_len, sink, B, T, H, S, Wt,
+                                    softmax_scale, out, as_stream(stream), who);
   }
   const size_t need = quant_attn_mfma_workspace(B * T, H, n_comp + Wt);
   if (need > 0 && (!ws || ws_bytes < need))

@@ -34,31 +34,18 @@ __device__ __forceinline__ void store4(void* p, int64_t i, float x, float y, flo
         make_uint2(f32_to_f16_bits(x) | (f32_to_f16_bits(y) << 16), f32_to_f16_bits(z) | (f32_to_f16_bits(w) << 16));
 }
 
-// Row i of the pieces' results -> row of the output and head of its sink (row % H): the same rows.
-struct SameRows {
-  __device__ int64_t operator()(uint32_t i, int& head, int H) const {
-    head = static_cast<int>(i) % H;
-    return i;
-  }
-};
-
 // Merges the source pieces of each (target, head) row: M = max(sink, piece maxima),
 // L = 2^(sink - M) + sum_p 2^(m_p - M) l_p, out = sum_p 2^(m_p - M) O_p / L (log2 units), as an
 // online merge over chunks of 8 pieces whose loads are all issued together.  D / 4 threads per
 // row, 4 dims each, NT / (D / 4) rows per workgroup (NT = 256, or 64 when that would leave CUs
 // without a workgroup, so that a call of few rows spreads its loads over as many CUs).
-// Map: which output row and sink head a row of pieces belongs to (negative: none).  DT, SDT: the
-// output's and the sink's types.
-template <int DT, int D, int NT, int SDT, typename Map>
+template <int DT, int D, int NT>
 __global__ __launch_bounds__(NT) void sink_attn_combine_kernel(const float* __restrict__ part, int n_split,
                                                                const void* __restrict__ sink, int sink_scalar,
-                                                               int H, int rows, void* __restrict__ out, Map map) {
+                                                               int H, int rows, void* __restrict__ out) {
   constexpr int kChunk = 8, kPer = D / 4, kStride = kPartStride<D>;
   const int row = static_cast<int>(blockIdx.x) * (NT / kPer) + static_cast<int>(threadIdx.x) / kPer;
   if (row >= rows) return;
-  int head;
-  const int64_t orow = map(static_cast<uint32_t>(row), head, H);
-  if (orow < 0) return;
   const int j = threadIdx.x % kPer;
   const float* p = part + static_cast<int64_t>(row) * n_split * kStride;
   float m[kChunk], l[kChunk];
@@ -75,7 +62,7 @@ __global__ __launch_bounds__(NT) void sink_attn_combine_kernel(const float* __re
       ml[i] = *reinterpret_cast<const float2*>(ps);
       o[i] = *reinterpret_cast<const f32x4_t*>(ps + 4 + 4 * j);
     }
-    if (sk) *sk = load_elem<SDT>(sink, sink_scalar ? 0 : head);
+    if (sk) *sk = load_elem<DT>(sink, sink_scalar ? 0 : row % H);
 #pragma unroll
     for (int i = 0; i < kChunk; ++i) asm volatile("" : "+v"(ml[i].x), "+v"(ml[i].y), "+v"(o[i]));
     if (sk) asm volatile("" : "+v"(*sk));
@@ -110,19 +97,19 @@ __global__ __launch_bounds__(NT) void sink_attn_combine_kernel(const float* __re
     }
   }
   const float r = den > 0.0f ? 1.0f / den : 0.0f;
-  store4<DT>(out, orow * D + 4 * j, acc[0] * r, acc[1] * r, acc[2] * r, acc[3] * r);
+  store4<DT>(out, static_cast<int64_t>(row) * D + 4 * j, acc[0] * r, acc[1] * r, acc[2] * r, acc[3] * r);
 }
 
 // Enqueues the combine of `rows` (target, head) rows of n_split pieces each.
-template <int DT, int D, int SDT = DT, typename Map = SameRows>
+template <int DT, int D>
 void launch_combine(const float* part, int n_split, const void* sink, int sink_scalar, int H, int64_t rows, void* out,
-                    hipStream_t st, Map map = Map{}) {
+                    hipStream_t st) {
   constexpr int kPer = D / 4;
   const bool wide = ceil_div(rows, static_cast<int64_t>(256 / kPer)) >= 256;
   const int nt = wide ? 256 : 64;
   const dim3 grid(static_cast<uint32_t>(ceil_div(rows, static_cast<int64_t>(nt / kPer))));
-  auto fn = wide ? sink_attn_combine_kernel<DT, D, 256, SDT, Map> : sink_attn_combine_kernel<DT, D, 64, SDT, Map>;
-  hipLaunchKernelGGL(fn, grid, dim3(nt), 0, st, part, n_split, sink, sink_scalar, H, static_cast<int>(rows), out, map);
+  auto fn = wide ? sink_attn_combine_kernel<DT, D, 256> : sink_attn_combine_kernel<DT, D, 64>;
+  hipLaunchKernelGGL(fn, grid, dim3(nt), 0, st, part, n_split, sink, sink_scalar, H, static_cast<int>(rows), out);
 }
 
 }  // namespace sinkc
