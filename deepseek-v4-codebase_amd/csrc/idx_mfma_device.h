@@ -1168,32 +1168,37 @@ __device__ __forceinline__ uint32_t select_row(const MfmaIdxArgs& a, const int b
     }
   } else {
     // Wave w takes the w-th contiguous part of the row.  First pass: keys > T are placed (in any
-    // order) and the part's keys == T counted; second pass: keys == T are placed in index order,
-    // after those of the waves before, until `need` of them are.  No barrier inside either pass.
+    // order) and the part's keys == T counted, or placed with them when every one of the row is taken;
+    // second pass, when some are not: keys == T are placed in index order, after those of the waves
+    // before, until `need` of them are.  No barrier inside either pass.
     // (Also for collected candidates with more keys == T than are taken: ranking those by index among
     // themselves compared every pair, 660 us for the 4096 zero scores of a 65536-key row.)
+    const bool all_eq = n_eq == need;
+    const uint32_t n_first = all_eq ? kk : n_gt;
     const int per = (n_vec + NW * 64 - 1) / (NW * 64) * 64;  // whole wave steps
     const int v0 = wv * per, v1 = min(n_vec, v0 + per);
     uint32_t eq = 0u;  // wave-uniform
 #pragma unroll 1
     for (int v = v0; v < v1; v += 64) {
       const u32x4_t kw = load_vec(v + lane);
-      uint32_t gt4 = 0u, eq_lane = 0u;  // bit e: key e > T; the lane's keys == T
+      uint32_t put4 = 0u, eq_lane = 0u;  // bit e: key e is placed; the lane's keys == T
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const bool in = 4 * (v + lane) + e < nv_i;
-        gt4 |= in && kw[e] > T ? 1u << e : 0u;
-        eq_lane += in && kw[e] == T ? 1u : 0u;
+        const bool in = 4 * (v + lane) + e < nv_i, is_eq = in && kw[e] == T;
+        put4 |= (in && kw[e] > T) || (all_eq && is_eq) ? 1u << e : 0u;
+        eq_lane += is_eq ? 1u : 0u;
       }
+      if (!all_eq) {
 #pragma unroll
-      for (int bit = 0; bit < 3; ++bit)
-        eq += static_cast<uint32_t>(__builtin_popcountll(__builtin_amdgcn_ballot_w64(((eq_lane >> bit) & 1u) != 0u))) << bit;
-      if (__builtin_amdgcn_ballot_w64(gt4 != 0u) == 0u) continue;  // wave-uniform
-      uint32_t pg = wave_reserve<3>(&s_cnt[0], static_cast<uint32_t>(__builtin_popcount(gt4)));
+        for (int bit = 0; bit < 3; ++bit)
+          eq += static_cast<uint32_t>(__builtin_popcountll(__builtin_amdgcn_ballot_w64(((eq_lane >> bit) & 1u) != 0u))) << bit;
+      }
+      if (__builtin_amdgcn_ballot_w64(put4 != 0u) == 0u) continue;  // wave-uniform
+      uint32_t pg = wave_reserve<3>(&s_cnt[0], static_cast<uint32_t>(__builtin_popcount(put4)));
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if ((gt4 >> e) & 1u) {
-          if (pg < n_gt) sel[pg] = sort_word(kw[e], static_cast<uint32_t>(4 * (v + lane) + e));
+        if ((put4 >> e) & 1u) {
+          if (pg < n_first) sel[pg] = sort_word(kw[e], static_cast<uint32_t>(4 * (v + lane) + e));
           ++pg;
         }
     }
@@ -1202,7 +1207,7 @@ __device__ __forceinline__ uint32_t select_row(const MfmaIdxArgs& a, const int b
     uint32_t run = 0u;  // keys == T before the current step
 #pragma unroll
     for (int w2 = 0; w2 < NW; ++w2) run += w2 < wv ? s_wave_eq[w2] : 0u;
-    for (int v = v0; v < v1 && run < need; v += 64) {  // wave-uniform; a lane's four keys are adjacent
+    for (int v = v0; v < v1 && run < need && !all_eq; v += 64) {  // wave-uniform; a lane's four keys are adjacent
       const u32x4_t kw = load_vec(v + lane);
       uint32_t m4 = 0u;
 #pragma unroll
