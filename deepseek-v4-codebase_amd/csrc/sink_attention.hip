@@ -417,8 +417,12 @@ __global__ __launch_bounds__(kThreads) void hca_compress_rows_kernel(const uint4
 }
 
 // Launches the kernel above when the row's entries fit (at most 4 entries per lane of a wave, else at
-// most 16 per lane of a workgroup) and the rows' threads fit one launch (the general kernel takes a
-// thread per column, fewer where rows are narrower than the team); false: nothing launched.
+// most 16 per lane of a workgroup), a row has at least two 16-byte pieces per lane of a wave, and the
+// rows' threads fit one launch; false: nothing launched.  Below two pieces, lanes of a row's wave only repeat
+// its last entry, and many rows wait for waves: bf16, 64 columns, general kernel / this one: 8 entries
+// (one piece) 4.0 / 5.4 us for 4096 rows and 26 / 27 for 32768; 16 entries 5.7 / 5.8 and 47 / 28.  32768 rows
+// of one entry of 8 columns: 2.5 / 49 us.  fp32, 64 columns: 4 entries 3.1 / 3.2 and 16 / 13 us, 8 entries 3.9 /
+// 3.4 and 27 / 22.
 template <int DT>
 bool launch_compress_rows(const void* c, const void* z, int64_t B, int64_t M, int64_t D, void* out, hipStream_t st) {
   const int64_t ncol = D * static_cast<int64_t>(dtype_size(DT)) / 16;
@@ -426,6 +430,7 @@ bool launch_compress_rows(const void* c, const void* z, int64_t B, int64_t M, in
       !is_aligned(c, 16) || !is_aligned(z, 16))
     return false;
   const int64_t wave_groups = 64 / ncol, wg_groups = 256 / ncol;
+  if (M < 2 * wave_groups) return false;
   const uint4* cv = static_cast<const uint4*>(c);
   const uint4* zv = static_cast<const uint4*>(z);
   auto go = [&](auto fn, int64_t grid) {
@@ -434,8 +439,7 @@ bool launch_compress_rows(const void* c, const void* z, int64_t B, int64_t M, in
                        static_cast<int>(ncol), out);
     return true;
   };
-  if (M <= wave_groups) return go(hca_compress_rows_kernel<DT, 1, 1>, ceil_div(B, int64_t(4)));
-  if (M <= 2 * wave_groups) return go(hca_compress_rows_kernel<DT, 2, 1>, ceil_div(B, int64_t(4)));
+  if (M == 2 * wave_groups) return go(hca_compress_rows_kernel<DT, 2, 1>, ceil_div(B, int64_t(4)));
   if (M <= 4 * wave_groups) return go(hca_compress_rows_kernel<DT, 4, 1>, ceil_div(B, int64_t(4)));
   if (M <= 4 * wg_groups) return go(hca_compress_rows_kernel<DT, 4, 4>, B);
   if (M <= 8 * wg_groups) return go(hca_compress_rows_kernel<DT, 8, 4>, B);

@@ -47,10 +47,23 @@ def test_infinities_stay_in_their_column(dev):
 
 
 def test_more_rows_than_a_launch_of_whole_waves(dev):
-    # 2^26 rows of 16 bytes: a wave each would be 2^32 work-items, past what a launch takes, so the call
-    # runs on the general kernel (one entry per row: the result is the row itself)
+    # 2^26 rows of 16 bytes: a wave each would be 2^32 work-items, past what a launch takes; the general
+    # kernel serves them (one entry per row: the result is the row itself)
     B, D = 1 << 26, 8
     c = torch.randint(-100, 100, (B, 1, D), device=dev, dtype=torch.int8).to(torch.bfloat16)
     z = torch.zeros_like(c)
     got = hca_compress(c, z)
     assert torch.equal(got, c[:, 0])
+
+
+# the line between the kernels: two 16-byte pieces per lane of a wave (128 pieces a row), one entry below and
+# above it, for the narrowest and the widest rows of the row kernel
+@pytest.mark.parametrize("dtype,M,D", [(torch.bfloat16, M, D) for M, D in ((127, 8), (128, 8), (129, 8), (15, 64), (16, 64),
+                                                                         (17, 64), (1, 512), (2, 512), (3, 512))]
+                         + [(torch.float32, M, D) for M, D in ((127, 4), (128, 4), (129, 4), (1, 256), (2, 256), (3, 256))])
+def test_line_between_the_kernels(dev, dtype, M, D):
+    g = torch.Generator().manual_seed(M * D)
+    c, z = torch.randn(5, M, D, generator=g).to(dtype), (torch.randn(5, M, D, generator=g) * 2).to(dtype)
+    tol = 1e-5 if dtype == torch.float32 else 5e-3
+    np.testing.assert_allclose(to_np_f32(hca_compress(c.to(dev), z.to(dev))), O.hca_compress(to_np_f32(c), to_np_f32(z)),
+                               rtol=tol, atol=tol)
