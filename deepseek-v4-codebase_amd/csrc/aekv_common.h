@@ -68,7 +68,8 @@ int sink_attention_mfma(const void* q, const void* kv, const void* idx, int idx_
 // The same in fp32 arithmetic (sink_attention_f32.hip): fp32 at head_dim 64 / 128, 16-bit at 64; q, kv and
 // out aligned to four elements.  A workspace that is too small or misaligned runs the call unsplit.
 bool sink_attention_f32_supported(int32_t dtype, int64_t D);
-bool sink_attention_f32_fits(bool dense, int64_t D, int64_t B, int64_t T, int64_t H, int64_t S, int64_t K);
+// (supported types and dims:) calls within its limits and not faster on the VALU kernel
+bool sink_attention_f32_takes(bool dense, int64_t D, int64_t B, int64_t T, int64_t H, int64_t S, int64_t K);
 size_t sink_attention_f32_workspace(bool dense, int64_t D, int64_t B, int64_t T, int64_t H, int64_t K);
 int sink_attention_f32(const void* q, const void* kv, const void* idx, int idx_kind, const void* sink, int sink_scalar,
                        int32_t dtype, int64_t B, int64_t T, int64_t H, int64_t D, int64_t S, int64_t K, float scale,

@@ -516,7 +516,7 @@ int sparse_common(const void* q, const void* kv, const void* topk, int idx_kind,
     return sink_attention_mfma(q, kv, topk, idx_kind, sink, scalar, dtype, B, T, H, S, K, scale, ws, ws_bytes, out, st,
                                who);
   const size_t quad = 4 * dtype_size(dtype);
-  if (sink_attention_f32_supported(dtype, D) && sink_attention_f32_fits(idx_kind == 0, D, B, T, H, S, K) &&
+  if (sink_attention_f32_supported(dtype, D) && sink_attention_f32_takes(idx_kind == 0, D, B, T, H, S, K) &&
       is_aligned(q, quad) && is_aligned(out, quad) && (K == 0 || is_aligned(kv, quad)))
     return sink_attention_f32(q, kv, topk, idx_kind, sink, scalar, dtype, B, T, H, D, S, K, scale, ws, ws_bytes, out,
                               st, who);
@@ -587,7 +587,7 @@ extern "C" size_t aekv_sink_attention_workspace_size(int32_t dtype, int64_t B, i
   if (!is_float_dtype(dtype) || B <= 0 || T <= 0 || H <= 0 || S < 0) return 0;
   if (sink_attention_f32_supported(dtype, D)) {
     const int64_t n = K < 0 ? S : K;
-    return sink_attention_f32_fits(K < 0, D, B, T, H, S, n) ? sink_attention_f32_workspace(K < 0, D, B, T, H, n) : 0;
+    return sink_attention_f32_takes(K < 0, D, B, T, H, S, n) ? sink_attention_f32_workspace(K < 0, D, B, T, H, n) : 0;
   }
   if (!sink_attention_mfma_supported(dtype, D)) return 0;
   return K < 0 ? sink_attention_mfma_workspace(true, B, T, H, S, S) : sink_attention_mfma_workspace(false, B, T, H, S, K);

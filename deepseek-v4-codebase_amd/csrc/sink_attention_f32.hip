@@ -6,8 +6,8 @@
 // aether_kernels/csrc/sparse_sink_attention_cuda.cu:47-114) and tiled_prefill_attention
 // (aether_kernels/sparse_attention.py:19-42), the sink counted once (aether_2b/modeling.py:158-178).
 //
-// What bounds it: the fp32 matrix rate (v_mfma_f32_16x16x4_f32, 64 products per cycle and SIMD) on
-// dense calls with many rows, memory latency on the others.  A workgroup owns 16 NQ query rows that
+// What bounds it: the fp32 matrix rate (v_mfma_f32_16x16x4_f32: 1024 multiply-adds in 32 cycles, 32 per
+// cycle and SIMD) on dense calls with many rows, memory latency on the others.  A workgroup owns 16 NQ query rows that
 // attend the same sources (consecutive (target, head) rows of a dense call, the heads of one target
 // of a sparse one); its NW waves take every NW-th group of 16 sources straight from global memory
 // into registers, in layouts that need no LDS and no lane exchange:
@@ -27,8 +27,8 @@
 // LDS; launches with few row blocks and many sources also split the sources over workgroups
 // (sink_combine.h).
 //
-// Measured (256 targets x 12 heads over 2176 fp32 sources, 128 dims): 46 us and a 4.5 us combine, 35x
-// the VALU kernel's 1.1 to 1.7 ms; the matrix cores are busy for 24 us of it (the loop runs 84% busy
+// Measured (256 targets x 12 heads over 2176 fp32 sources, 128 dims): 46 us and a 4.5 us combine, where
+// the VALU kernel took 1.1 to 1.7 ms (22x to 34x); the matrix cores are busy for 24 us of it (the loop runs 84% busy
 // with two waves per SIMD, the rest is the first and last memory rounds and the waves' merge).
 // 128 targets x 16 heads over 64 picked sources: 6.4 us (40.7); one target over 2176: 12 + 4 us (677).
 #include <algorithm>
@@ -354,6 +354,13 @@ struct F32Plan {
 // workgroups.  Splits start above 40 groups (640 sources) when the workgroups leave CUs idle: one
 // target over 656 sources takes 11.4 us and a 4 us combine instead of 18.8 us; pieces fill the chip
 // (512 four-wave workgroups or 256 of eight) and keep at least two groups per wave.
+// Sparse calls of at most eight groups and six heads take one wave per workgroup once those fill half the chip:
+// with so few of a product's 16 rows in use, the merge of four waves' 16 rows (one to three of them without a
+// group at few sources) left the VALU kernel ahead.  VALU / four waves / one, fp32: 4096 targets x 4 heads x 128
+// dims over 16 sources 51 / 35 / 14.7 us, over one 19.5 / 27.9 / 12.4; 16384 targets of one head x 128 dims over 64
+// 129 / 173 / 104, x 64 dims over 16 26.0 / 39.4 / 20.8; 1024 targets of one head x 64 dims over 64 21 / 7.0 / 6.6;
+// 512 over 64 20.8 / 5.1 / 6.1.  One wave sums its groups in sequence: fp32 error against 64 bits over 64 / 128
+// sources 2.2e-7 / 2.8e-7, four waves 1.9e-7 / 2.1e-7, the VALU kernel 2.8e-7 / 3.3e-7 (64 dims).
 F32Plan f32_plan(bool dense, int64_t D, int64_t B, int64_t T, int64_t H, int64_t K, bool may_split) {
   F32Plan p{};
   const int64_t shared = dense ? T * H : H, units = dense ? B : B * T;
@@ -361,9 +368,9 @@ F32Plan f32_plan(bool dense, int64_t D, int64_t B, int64_t T, int64_t H, int64_t
   const bool split = may_split && groups > 40;
   const int64_t blocks2 = units * ceil_div(shared, int64_t(32));
   p.nq = dense && blocks2 >= (split ? 36 : 256) ? 2 : 1;
-  p.nw = p.nq == 1 && groups >= 16 ? 8 : 4;
   p.n_blk = ceil_div(shared, static_cast<int64_t>(16 * p.nq));
   p.wgs = units * p.n_blk;
+  p.nw = p.nq == 1 && groups >= 16 ? 8 : !dense && H <= 6 && groups <= 8 && p.wgs >= 1024 ? 1 : 4;
   p.n_split = 1;
   const int64_t fill = p.nw == 8 ? 256 : 512;
   if (split && p.wgs > 0)
@@ -380,6 +387,12 @@ void launch_f32(const SinkF32Args& a, const F32Plan& p, hipStream_t st) {
   if constexpr (IDX == 0) {
     if (p.nq == 2) {
       hipLaunchKernelGGL((sink_attn_f32_kernel<DT, D, 0, 2, 4>), grid, dim3(256), 0, st, a);
+      return;
+    }
+  }
+  if constexpr (IDX != 0) {
+    if (p.nw == 1) {
+      hipLaunchKernelGGL((sink_attn_f32_kernel<DT, D, IDX, 1, 1>), grid, dim3(64), 0, st, a);
       return;
     }
   }
@@ -402,7 +415,12 @@ bool sink_attention_f32_supported(int32_t dtype, int64_t D) {
   return dtype == AEKV_F32 ? (D == 64 || D == 128) : D == 64;
 }
 
-bool sink_attention_f32_fits(bool dense, int64_t D, int64_t B, int64_t T, int64_t H, int64_t S, int64_t K) {
+bool sink_attention_f32_takes(bool dense, int64_t D, int64_t B, int64_t T, int64_t H, int64_t S, int64_t K) {
+  // Many targets of one or two heads over a few sources: 15 or 14 of the 16 rows of a product are empty, and
+  // the VALU kernel's wave per row is the faster one.  VALU / this kernel, fp32, one head: 4096 targets x 64 dims
+  // over one source 5.2 / 6.9 us, over 16 10.6 / 7.3; x 128 dims 7.4 / 11.0 and 20 / 13; 16384 targets x 64 dims 11.7 /
+  // 19.9 and 26 / 20.8, x 128 dims 22 / 38 and 50 / 45; 2048 x 128 dims over one 5.5 / 6.4; 1024 targets equal.
+  if (!dense && H <= 2 && H * H * K <= 12 && B * T >= 2048 && H * H * K * 512 <= B * T) return false;
   const int64_t lim = 0x7fffffff - 4096;  // (32-bit positions, a few groups past the end among them)
   if (S > lim || K > lim || B * T * H > lim || T * H > lim) return false;
   // (256 or 512 threads per 16 or 32 rows, where the VALU kernel takes 64 per row: sparse calls of many

@@ -112,7 +112,7 @@ def test_more_targets_than_a_launch_of_whole_workgroups(dev):
     g = torch.Generator(device=dev).manual_seed(3)
     q = torch.randn(1, T, 1, D, generator=g, device=dev, dtype=torch.bfloat16)
     kv = torch.randn(1, S, 2, D, generator=g, device=dev, dtype=torch.bfloat16)
-    idx = torch.randint(0, S, (1, T, 2), generator=g, device=dev, dtype=torch.int32)
+    idx = torch.randint(0, S, (1, T, 130), generator=g, device=dev, dtype=torch.int32)
     sink = torch.zeros(1, device=dev, dtype=torch.bfloat16)
     got = sparse_sink_attention(q, kv, idx, sink, D ** -0.5)
     for lo in (0, T // 2, T - 4096):
@@ -120,3 +120,23 @@ def test_more_targets_than_a_launch_of_whole_workgroups(dev):
         want = sparse_sink_attention(q[:, part].contiguous(), kv, idx[:, part].contiguous(), sink, D ** -0.5)
         # both in fp32 from the same inputs: at most one bf16 rounding apart
         torch.testing.assert_close(got[:, part], want, rtol=2 ** -7, atol=1e-5)
+
+
+# Sparse calls either side of the lines between the VALU kernel, one wave and four waves per workgroup (targets,
+# heads, sources), none of them at all, and two head groups of a target.
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 64), (torch.float32, 128), (torch.bfloat16, 64)])
+@pytest.mark.parametrize("T,H,K", [(1023, 3, 128), (1024, 3, 128), (1024, 3, 129), (1025, 6, 1), (1025, 7, 1), (513, 17, 1), (2047, 1, 4), (2048, 1, 4),
+                                   (2048, 1, 5), (6144, 1, 12), (6144, 1, 13), (6143, 2, 3), (6144, 2, 3), (6144, 2, 4),
+                                   (3000, 1, 0)])
+def test_lines_between_kernels(dev, dtype, D, T, H, K):
+    g = torch.Generator(device=dev).manual_seed(T + H + K)
+    q = torch.randn(1, T, H, D, generator=g, device=dev).to(dtype)
+    kv = torch.randn(1, 300, 2, D, generator=g, device=dev).to(dtype)
+    idx = torch.randint(-20, 320, (1, T, K), generator=g, device=dev)  # some skipped
+    sink = torch.randn(H, generator=g, device=dev).to(dtype)
+    got = sparse_sink_attention(q, kv, idx, sink, D ** -0.5)
+    for lo in (0, T // 2, T - 100):
+        part = slice(lo, lo + 100)
+        want = O.sink_attention(to_np_f32(q[:, part]), to_np_f32(kv), idx[:, part].cpu().numpy(), to_np_f32(sink), D ** -0.5,
+                                threads=8)
+        np.testing.assert_allclose(to_np_f32(got[:, part]), want, rtol=_tol(dtype), atol=_tol(dtype))
