@@ -1,5 +1,6 @@
-"""The fast encode of D = 64 and 128 from every input type, bit for bit against the generic kernel (which
-the oracle pins), and the 4-element decode layout of fp32 outputs against the oracle."""
+"""The fast encodes of D = 64 and 128 from bf16 and fp16, bit for bit against the generic kernel (which the
+oracle pins); the encode of fp32 inputs, which has the generic kernel alone, against the oracle on the same
+vectors; and the 4-element decode layout of fp32 outputs against the oracle."""
 from __future__ import annotations
 
 import numpy as np
@@ -24,6 +25,12 @@ def _both(pq, x):
 
 
 def _same(pq, x):
+    if x.dtype == torch.float32:
+        codes, scale = pq.encode(x)
+        want_c, want_s = O.encode(x.cpu().numpy(), "f32", pq.bits, O.diag(42, x.shape[-1]))
+        np.testing.assert_array_equal(codes.cpu().numpy(), want_c)
+        np.testing.assert_array_equal(scale.cpu().numpy(), want_s)
+        return
     (cg, sg), (cf, sf) = _both(pq, x)
     assert torch.equal(cg, cf)
     assert torch.equal(sg.view(torch.int32), sf.view(torch.int32))  # (bits: NaN scales compare too)
@@ -53,9 +60,10 @@ def test_ties(dev, dtype, bits, d):
     _same(PolarQuant(bits), (x * 0.1).to(dtype).to(dev))  # rounded inputs: near ties
 
 
-# zero, tiny and huge vectors, infinities and NaN, and (fp32) sums that overflow, between ordinary vectors of one wave
-# (the 4-bit D = 128 bf16 kernel is another one, which takes finite vectors of ordinary range)
-@pytest.mark.parametrize("dtype,bits,d", [c for c in CASES if c != (torch.bfloat16, 4, 128)])
+# zero, tiny and huge vectors, infinities and NaN, and (bf16) sums that overflow, between ordinary vectors of one wave.
+# (The oracle converts a NaN ratio to a whole number, which C leaves undefined: fp32 vectors with one are left out.
+# The 4-bit D = 128 bf16 kernel is another one, which takes finite vectors of ordinary range: zero and tiny ones.)
+@pytest.mark.parametrize("dtype,bits,d", CASES)
 def test_extreme_vectors(dev, dtype, bits, d):
     x = torch.randn(64, d, generator=torch.Generator().manual_seed(d))
     big = 6e4 if dtype == torch.float16 else 3e38
@@ -72,8 +80,13 @@ def test_extreme_vectors(dev, dtype, bits, d):
     if dtype != torch.float16:
         x[30] *= 1e31  # above the fast quantiser's range, sums still finite
         x[31] *= 1e-36
+    if dtype == torch.float32:
+        x = x[[i for i in range(64) if i not in (22, 40, 41, 50, 51, 60)]]
+    elif (dtype, bits, d) == (torch.bfloat16, 4, 128):
+        x = x[:20]
     for rows in (slice(0, 16), slice(16, 35), slice(0, 64)):
-        _same(PolarQuant(bits), x[rows].to(dtype).to(dev))
+        if len(x[rows]):
+            _same(PolarQuant(bits), x[rows].to(dtype).to(dev))
 
 
 @pytest.mark.parametrize("bits", [4, 8])
