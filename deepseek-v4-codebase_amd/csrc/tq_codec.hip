@@ -107,8 +107,8 @@ __device__ __forceinline__ void store_decoded(uint8_t* o, const float (&a)[EPL])
 
 // Decode kernel: codes * scale -> WHT -> * diag -> out dtype.  PP == 0: a grid-stride loop.  PP > 0: PP
 // consecutive groups of 64 / LPV vectors per wave, all their loads issued first, no loop (the launch covers
-// every group), and stores past the caches.
-template <int BITS, int D, int ODT, int PP>
+// every group); NT: with stores past the caches.
+template <int BITS, int D, int ODT, int PP, bool NT>
 __global__ __launch_bounds__(kThreads) void tq_decode_kernel(const void* __restrict__ codes,
                                                              const float* __restrict__ scale, int64_t n_vec,
                                                              const float* __restrict__ diag, float c,
@@ -143,7 +143,7 @@ __global__ __launch_bounds__(kThreads) void tq_decode_kernel(const void* __restr
     for (int i = 0; i < PP; ++i) {
       float a[EPL];
       decode_lane_bytes<BITS, D, true, EPL>(w[i], s[i], sub, dg, c, a);
-      if (v0 + i * VPW < n_vec) store_decoded<ODT, EPL, true>(ob + (v0 + i * VPW) * OB, a);
+      if (v0 + i * VPW < n_vec) store_decoded<ODT, EPL, NT>(ob + (v0 + i * VPW) * OB, a);
     }
     return;
   }
@@ -196,37 +196,43 @@ fwd_fn pick_fwd_dt(int dt, int d) {
 template <int BITS, int ODT>
 dec_fn pick_dec(int d) {
   switch (d) {
-    case 1: return BITS == 4 ? nullptr : tq_decode_kernel<BITS, 1, ODT, 0>;
-    case 2: return tq_decode_kernel<BITS, 2, ODT, 0>;
-    case 4: return tq_decode_kernel<BITS, 4, ODT, 0>;
-    case 8: return tq_decode_kernel<BITS, 8, ODT, 0>;
-    case 16: return tq_decode_kernel<BITS, 16, ODT, 0>;
-    case 32: return tq_decode_kernel<BITS, 32, ODT, 0>;
-    case 64: return tq_decode_kernel<BITS, 64, ODT, 0>;
-    case 128: return tq_decode_kernel<BITS, 128, ODT, 0>;
-    case 256: return tq_decode_kernel<BITS, 256, ODT, 0>;
-    case 512: return tq_decode_kernel<BITS, 512, ODT, 0>;
+    case 1: return BITS == 4 ? nullptr : tq_decode_kernel<BITS, 1, ODT, 0, false>;
+    case 2: return tq_decode_kernel<BITS, 2, ODT, 0, false>;
+    case 4: return tq_decode_kernel<BITS, 4, ODT, 0, false>;
+    case 8: return tq_decode_kernel<BITS, 8, ODT, 0, false>;
+    case 16: return tq_decode_kernel<BITS, 16, ODT, 0, false>;
+    case 32: return tq_decode_kernel<BITS, 32, ODT, 0, false>;
+    case 64: return tq_decode_kernel<BITS, 64, ODT, 0, false>;
+    case 128: return tq_decode_kernel<BITS, 128, ODT, 0, false>;
+    case 256: return tq_decode_kernel<BITS, 256, ODT, 0, false>;
+    case 512: return tq_decode_kernel<BITS, 512, ODT, 0, false>;
     default: return nullptr;
   }
 }
 
 constexpr int kDecPasses = 4;
-// Codes and output together from which a decode streams (D = 64 and 128).  Measured, loop / streamed, on codes
-// coming round from three sets: 64 M elements to fp32 74 to 80 / 45 to 49 us (8-bit D = 64: 4.6 / 7.0 TB/s), 64 M
-// to bf16 8-bit 39 to 40 / 31, 100 M to fp16 60 to 66 / 46 to 54, 403 M to bf16 8-bit D = 64 234 / 207; 32 M to
-// fp32 (151 to 168 MB) 24 to 27 / 25 to 28, below that within the noise: the loop's output then stays in the caches.
+// Codes and output together from which a decode streams (D = 64 and 128), and from which its stores go past
+// the caches.  Measured on codes coming round from two sets, loop / streamed / streamed past the caches, the
+// decode alone and with a caller's pass that reads the decoded tensor (a product with four columns):
+//   fp32, 8-bit D = 128   170 MB 29 / 27 / 26 and 69 / 66 / 74 us    300 MB 60 / 47 / 44 and 121 / 108 / 118
+//                         400 MB 82 / 71 / 57 and 181 / 167 / 157    600 MB 120 / 105 / 86 and 261 / 239 / 227
+//   bf16, 8-bit D = 128   170 MB 30 / 27 / 27 and 71 / 70 / 78 us    300 MB 59 / 50 / 46 and 115 / 107 / 123
+//                         400 MB 80 / 70 / 67 and 162 / 153 / 150    600 MB 113 / 103 / 101 and 249 / 240 / 238
+// Up to about 1.5 times the Infinity Cache a reader gains more from an output that is still there than the
+// decode loses by it.  Below 160 MB the loop and the streams are within the noise of each other.
 constexpr int64_t kDecStreamBytes = 160000000;
+constexpr int64_t kDecPastCachesBytes = 400000000;
 
-template <int BITS, int ODT>
+template <int BITS, int ODT, bool NT>
 dec_fn pick_dec_stream(int d) {
-  return d == 128 ? tq_decode_kernel<BITS, 128, ODT, kDecPasses> : tq_decode_kernel<BITS, 64, ODT, kDecPasses>;
+  return d == 128 ? tq_decode_kernel<BITS, 128, ODT, kDecPasses, NT> : tq_decode_kernel<BITS, 64, ODT, kDecPasses, NT>;
 }
 
-template <int BITS>
+template <int BITS, bool NT>
 dec_fn pick_dec_stream_dt(int odt, int d) {
-  if (odt == AEKV_F32) return pick_dec_stream<BITS, AEKV_F32>(d);
-  if (odt == AEKV_F16) return pick_dec_stream<BITS, AEKV_F16>(d);
-  return pick_dec_stream<BITS, AEKV_BF16>(d);
+  if (odt == AEKV_F32) return pick_dec_stream<BITS, AEKV_F32, NT>(d);
+  if (odt == AEKV_F16) return pick_dec_stream<BITS, AEKV_F16, NT>(d);
+  return pick_dec_stream<BITS, AEKV_BF16, NT>(d);
 }
 
 template <int BITS>
@@ -309,7 +315,9 @@ extern "C" int aekv_tq_decode(const void* codes, const float* scale, int64_t n_v
   const int64_t blocks = ceil_div(n_vec, static_cast<int64_t>(kDecPasses) * (kThreads / 64) * (64 / (d / lane_el)));
   const int64_t bytes = n_vec * d * static_cast<int64_t>(dtype_size(out_dtype)) + n_vec * d * bits / 8;
   if (use_specialised_codec() && (d == 64 || d == 128) && bytes >= kDecStreamBytes && blocks <= 0x7fffffff) {
-    dec_fn fn = bits == 8 ? pick_dec_stream_dt<8>(out_dtype, d) : pick_dec_stream_dt<4>(out_dtype, d);
+    const bool past = bytes >= kDecPastCachesBytes;
+    dec_fn fn = bits == 8 ? (past ? pick_dec_stream_dt<8, true>(out_dtype, d) : pick_dec_stream_dt<8, false>(out_dtype, d))
+                          : (past ? pick_dec_stream_dt<4, true>(out_dtype, d) : pick_dec_stream_dt<4, false>(out_dtype, d));
     hipLaunchKernelGGL(fn, dim3(static_cast<uint32_t>(blocks)), dim3(kThreads), 0, as_stream(stream), codes, scale, n_vec,
                        diag, wht_scale(d), out);
     return check_launch("aekv_tq_decode");

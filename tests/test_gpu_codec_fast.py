@@ -103,12 +103,13 @@ def test_decode_to_fp32(dev, bits, d):
         np.testing.assert_array_equal(got.cpu().numpy(), O.decode(codes, scale, bits, O.diag(42, d), "f32"))
 
 
-# decodes past the caches (160 MB of codes and output), with a last wave and group partly filled
+# streamed decodes (160 MB of codes and output; 400 MB: past the caches), with a last wave and group partly filled
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("bits,d", [(4, 64), (8, 64), (4, 128), (8, 128)])
-def test_streamed_decode(dev, dtype, bits, d):
+@pytest.mark.parametrize("line", [160_000_000, 400_000_000])
+def test_streamed_decode(dev, dtype, bits, d, line):
     es = 4 if dtype == torch.float32 else 2
-    n = -(-160_000_000 // (d * es + d * bits // 8)) + 37
+    n = -(-line // (d * es + d * bits // 8)) + 37
     g = torch.Generator(device=dev).manual_seed(n + bits)
     lo, hi = (0, 256) if bits == 4 else (-127, 128)
     codes = torch.randint(lo, hi, (n, d * bits // 8), generator=g, device=dev, dtype=torch.uint8 if bits == 4 else torch.int8)
