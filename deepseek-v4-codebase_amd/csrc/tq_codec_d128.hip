@@ -764,10 +764,18 @@ fast_enc_fn pick_fast(int bits, int d, int& vpw) {
 
 }  // namespace
 
-// Launches the fast encode; false when the shape, the type or the alignment is not one of its own.
+// fp16 elements from which the fast encode is the faster one: a wave takes 16 or 32 vectors where the generic
+// kernel's takes 4 or 8, so that a small call leaves most of the chip idle and waits for one wave's chain.
+// Generic / fast, 8-bit D = 128: 100 vectors 2.45 / 3.2 us, 8192 3.5 / 4.4, 16384 4.6 / 4.7, 32768 6.2 / 5.8, 65536
+// 10.2 / 7.5; 4-bit D = 64: 100 vectors 2.3 / 2.6, 16384 3.4 / 4.1, 32768 4.3 / 4.4, 65536 6.0 / 5.2.
+// (bf16, whose fast kernel needs no conversion, takes it at every size.)
+constexpr int64_t kFastF16Elements = int64_t(3) << 20;
+
+// Launches the fast encode; false when the shape, the type, the size or the alignment is not one of its own.
 bool launch_encode_fast(const void* x, int x_dtype, int64_t n_vec, int bits, int d, const float* diag, float c,
                         void* codes, float* scale, hipStream_t st) {
   if (!is_aligned(x, 16) || !is_aligned(codes, 16) || (d != 64 && d != 128)) return false;
+  if (x_dtype == AEKV_F16 && n_vec * d < kFastF16Elements) return false;
   int vpw = 0;
   const fast_enc_fn kern = x_dtype == AEKV_BF16  ? pick_fast<AEKV_BF16>(bits, d, vpw)
                            : x_dtype == AEKV_F16 ? pick_fast<AEKV_F16>(bits, d, vpw)

@@ -31,6 +31,10 @@ def _same(pq, x):
         np.testing.assert_array_equal(codes.cpu().numpy(), want_c)
         np.testing.assert_array_equal(scale.cpu().numpy(), want_s)
         return
+    if x.dtype == torch.float16:  # (the fast fp16 encode starts at 3 * 2^20 elements: whole waves ahead of x)
+        ahead = torch.randn((3 << 20) // x.shape[-1], x.shape[-1], generator=torch.Generator(device=x.device).manual_seed(0),
+                            device=x.device)
+        x = torch.cat([ahead.to(x.dtype), x])
     (cg, sg), (cf, sf) = _both(pq, x)
     assert torch.equal(cg, cf)
     assert torch.equal(sg.view(torch.int32), sf.view(torch.int32))  # (bits: NaN scales compare too)
@@ -87,6 +91,17 @@ def test_extreme_vectors(dev, dtype, bits, d):
     for rows in (slice(0, 16), slice(16, 35), slice(0, 64)):
         if len(x[rows]):
             _same(PolarQuant(bits), x[rows].to(dtype).to(dev))
+
+
+# the fp16 line between the generic and the fast encode: either side of 3 * 2^20 elements
+@pytest.mark.parametrize("bits,d", [(4, 64), (8, 64), (4, 128), (8, 128)])
+def test_fp16_line(dev, bits, d):
+    n = (3 << 20) // d
+    x = normal_with_outliers((n, d), d + bits, dtype=torch.float16, trailing_dims=1).to(dev)
+    pq = PolarQuant(bits)
+    for rows in (n - 1, n):
+        (cg, sg), (cf, sf) = _both(pq, x[:rows])
+        assert torch.equal(cg, cf) and torch.equal(sg, sf)
 
 
 @pytest.mark.parametrize("bits", [4, 8])
