@@ -183,13 +183,14 @@ def on_device(device: torch.device):
 # always gets a buffer of its own, from the graph's private pool: its replays keep the address, while
 # a cached buffer is replaced when a larger call comes and belongs to the eager calls of its stream.
 _ws_cache: dict = {}
+_capturing = getattr(torch._C, "_cuda_isCurrentStreamCapturing", torch.cuda.is_current_stream_capturing)
 
 
 def workspace(nbytes: int, device: torch.device, stream: int) -> Optional[torch.Tensor]:
     """A buffer of at least nbytes for a call on `stream`, the current stream of the current device."""
     if nbytes <= 0:
         return None
-    if torch.cuda.is_current_stream_capturing():
+    if _capturing():
         return torch.empty(nbytes, dtype=torch.uint8, device=device)
     key = (device.index, stream)
     buf = _ws_cache.get(key)

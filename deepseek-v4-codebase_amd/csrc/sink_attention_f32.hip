@@ -346,12 +346,15 @@ struct F32Plan {
   size_t ws;
 };
 
-// Rows of a workgroup, its waves, and the source pieces.  Measured with 12 heads over 2176 fp32
-// sources of 128 dims (kernel alone; one row group of 8 waves against two of 4): 43 targets 16.0
-// against 19.7 us, 86 targets 23.9 against 24.9, 171 targets 52.1 against 34.8 (two groups read each
-// source half as often, and four waves leave more pieces to split into).  Calls that are not split
-// (256 targets over 300 sources: 14.0 against 17.9 us) keep one group until the chip is full of
-// workgroups.  Splits start above 40 groups (640 sources) when the workgroups leave CUs idle: one
+// Rows of a workgroup, its waves, and the source pieces.  One row group of 8 waves against two of 4 (which
+// read each source half as often, and leave more pieces to split into), 12 heads, kernel and combine.  Split
+// calls take two from 65 blocks of 32 rows, where one group's blocks are more than 128 and no longer split: over
+// 2176 sources, fp32, 128 dims, 57 blocks 31.6 / 33.4 us, 65 50 / 35.6, 96 50 / 45.5 (113 50 / 54, 150 96 / 67: the
+// rounds of a full chip alternate); 64 dims 57 blocks 18.3 / 20.3, 65 27.6 / 21.4; bf16 19.9 / 21.1 and 30.7 /
+// 22.3; over 1003 sources 20.3 / 24.5 and 27.3 / 25.4 (fp32, 128 dims).  Calls that are not split take two from 256
+// blocks: over 300 sources 96 blocks 13.4 / 17.9, 257 34 / 28, 64 dims 257 16.4 / 16.7, 512 22.1 / 18.1 (at 128
+// dims two are ahead from 150 blocks already, 24.5 / 18.1; over 600 sources x 64 dims 257 blocks take 25 / 29).
+// Splits start above 40 groups (640 sources) when the workgroups leave CUs idle: one
 // target over 656 sources takes 11.4 us and a 4 us combine instead of 18.8 us; pieces fill the chip
 // (512 four-wave workgroups or 256 of eight) and keep at least two groups per wave.
 // Sparse calls of at most eight groups and six heads take one wave per workgroup once those fill half the chip:
@@ -367,7 +370,7 @@ F32Plan f32_plan(bool dense, int64_t D, int64_t B, int64_t T, int64_t H, int64_t
   const int64_t groups = ceil_div(K, static_cast<int64_t>(kSrc));
   const bool split = may_split && groups > 40;
   const int64_t blocks2 = units * ceil_div(shared, int64_t(32));
-  p.nq = dense && blocks2 >= (split ? 36 : 256) ? 2 : 1;
+  p.nq = dense && blocks2 >= (split ? 65 : 256) ? 2 : 1;
   p.n_blk = ceil_div(shared, static_cast<int64_t>(16 * p.nq));
   p.wgs = units * p.n_blk;
   p.nw = p.nq == 1 && groups >= 16 ? 8 : !dense && H <= 6 && groups <= 8 && p.wgs >= 1024 ? 1 : 4;

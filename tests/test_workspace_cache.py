@@ -16,7 +16,7 @@ from aetherkv.decode import attention_workspace, decode_workspace, indexer_works
 def test_captured_calls_get_buffers_of_their_own(monkeypatch):
     monkeypatch.setattr(L, "_ws_cache", {})
     capturing = [False]
-    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    monkeypatch.setattr(L, "_capturing", lambda: capturing[0])
     cpu = torch.device("cpu")
     eager = L.workspace(1000, cpu, 7)
     assert L.workspace(600, cpu, 7) is eager  # reused
