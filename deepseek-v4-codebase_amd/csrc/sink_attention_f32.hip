@@ -348,15 +348,16 @@ struct F32Plan {
 
 // Rows of a workgroup, its waves, and the source pieces.  One row group of 8 waves against two of 4 (which
 // read each source half as often, and leave more pieces to split into), 12 heads, kernel and combine.  Split
-// calls take two from 65 blocks of 32 rows, where one group's blocks are more than 128 and no longer split: over
-// 2176 sources, fp32, 128 dims, 57 blocks 31.6 / 33.4 us, 65 50 / 35.6, 96 50 / 45.5 (113 50 / 54, 150 96 / 67: the
-// rounds of a full chip alternate); 64 dims 57 blocks 18.3 / 20.3, 65 27.6 / 21.4; bf16 19.9 / 21.1 and 30.7 /
-// 22.3; over 1003 sources 20.3 / 24.5 and 27.3 / 25.4 (fp32, 128 dims).  Calls that are not split take two from 256
-// blocks: over 300 sources 96 blocks 13.4 / 17.9, 257 34 / 28, 64 dims 257 16.4 / 16.7, 512 22.1 / 18.1 (at 128
-// dims two are ahead from 150 blocks already, 24.5 / 18.1; over 600 sources x 64 dims 257 blocks take 25 / 29).
-// Splits start above 40 groups (640 sources) when the workgroups leave CUs idle: one
-// target over 656 sources takes 11.4 us and a 4 us combine instead of 18.8 us; pieces fill the chip
-// (512 four-wave workgroups or 256 of eight) and keep at least two groups per wave.
+// calls take two from 65 blocks of 32 rows, where one group's blocks are more than 128 and no longer split:
+// over 2176 sources, fp32, 128 dims, 57 blocks 31.6 / 33.4 us, 65 50 / 35.6, 96 50 / 45.5 (113 50 / 54, 150 96
+// / 67: the rounds of a full chip alternate); 64 dims 57 blocks 18.3 / 20.3, 65 27.6 / 21.4; bf16 19.9 / 21.1
+// and 30.7 / 22.3; over 1003 sources 20.3 / 24.5 and 27.3 / 25.4 (fp32, 128 dims).  Below 56 groups the line
+// is 36: over 700 sources 41 blocks 17.7 / 16.0, 48 18.0 / 16.4 (57 to 128 blocks 19 to 21 / 23 to 28, 150 40
+// / 32.5).  Calls that are not split take two from 256 blocks: over 300 sources 96 blocks 13.4 / 17.9, 257 34
+// / 28, 64 dims 257 16.4 / 16.7, 512 22.1 / 18.1 (at 128 dims two are ahead from 150 blocks already, 24.5 /
+// 18.1; over 600 sources x 64 dims 257 blocks take 25 / 29). Splits start above 40 groups (640 sources) when
+// the workgroups leave CUs idle: one target over 656 sources takes 11.4 us and a 4 us combine instead of 18.8
+// us; pieces fill the chip (512 four-wave workgroups or 256 of eight) and keep at least two groups per wave.
 // Sparse calls of at most eight groups and six heads take one wave per workgroup once those fill half the chip:
 // with so few of a product's 16 rows in use, the merge of four waves' 16 rows (one to three of them without a
 // group at few sources) left the VALU kernel ahead.  VALU / four waves / one, fp32: 4096 targets x 4 heads x 128
@@ -370,7 +371,7 @@ F32Plan f32_plan(bool dense, int64_t D, int64_t B, int64_t T, int64_t H, int64_t
   const int64_t groups = ceil_div(K, static_cast<int64_t>(kSrc));
   const bool split = may_split && groups > 40;
   const int64_t blocks2 = units * ceil_div(shared, int64_t(32));
-  p.nq = dense && blocks2 >= (split ? 65 : 256) ? 2 : 1;
+  p.nq = dense && blocks2 >= (!split ? 256 : groups < 56 ? 36 : 65) ? 2 : 1;
   p.n_blk = ceil_div(shared, static_cast<int64_t>(16 * p.nq));
   p.wgs = units * p.n_blk;
   p.nw = p.nq == 1 && groups >= 16 ? 8 : !dense && H <= 6 && groups <= 8 && p.wgs >= 1024 ? 1 : 4;
