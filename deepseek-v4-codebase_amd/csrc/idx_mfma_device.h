@@ -1092,42 +1092,52 @@ __device__ __forceinline__ uint32_t select_row(const MfmaIdxArgs& a, const int b
         if (lvl == 0 || (key >> shift) == prefix) atomicAdd(&h[(key >> nshift) & mask], 1u);
       }
     } else {
-      // Rows come here because many keys are equal, or because they have fewer slots than k and too
-      // many keys for the candidates' LDS (NT = 512: 1537 to 16 k keys).  Where a quarter of a wave's
-      // first keys meet in one bin, the bin of each element's first counted key takes one atomic for all
-      // of its lanes there; elsewhere each key takes its own (aggregated throughout, a row of 3000
-      // distinct keys took 1 us longer).
+      auto counted = [&](const uint32_t key, const int at) {
+        return at < nv_i && (lvl == 0 || (key >> shift) == prefix);
+      };
+      // The bin of the wave's first counted key takes one atomic for all of its lanes there.
+      auto count_together = [&](const uint32_t key, const int at) {
+        const bool act = counted(key, at);
+        const uint64_t am = __builtin_amdgcn_ballot_w64(act);
+        if (am == 0u) return;  // wave-uniform
+        const uint32_t bin = (key >> nshift) & mask;
+        const int first = __builtin_ctzll(am);
+        const uint32_t b0 = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(bin), first));
+        const uint64_t same = __builtin_amdgcn_ballot_w64(act && bin == b0);
+        if (lane == first) atomicAdd(&h[b0], static_cast<uint32_t>(__builtin_popcountll(same)));
+        if (act && bin != b0) atomicAdd(&h[bin], 1u);
+      };
+      if (static_cast<int64_t>(kk) > n_slots) {
+        // A row with fewer slots than k, and too many keys for the candidates' LDS (NT = 512: 1537 to 16 k):
+        // mostly distinct keys, an atomic each, unless a quarter of the wave's first keys meet in one bin
+        // (counted together throughout, 3000 distinct keys took 1 us longer).
 #pragma unroll 1
-      for (int v = 64 * wv; v < n_vec; v += NT) {
-        const u32x4_t kw = load_vec(v + lane);
-        bool act[4];
-        uint32_t bin[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          act[e] = 4 * (v + lane) + e < nv_i && (lvl == 0 || (kw[e] >> shift) == prefix);
-          bin[e] = (kw[e] >> nshift) & mask;
-        }
-        auto first_bin = [&](int e, uint64_t am) {  // bin of the first lane of am
-          return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(bin[e]), __builtin_ctzll(am)));
-        };
-        const uint64_t am0 = __builtin_amdgcn_ballot_w64(act[0]);
-        bool meet = false;  // wave-uniform
-        if (am0 != 0u) {
-          const uint32_t b0 = first_bin(0, am0);
-          meet = __builtin_popcountll(__builtin_amdgcn_ballot_w64(act[0] && bin[0] == b0)) >= 16;
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          if (!meet) {
-            if (act[e]) atomicAdd(&h[bin[e]], 1u);
-            continue;
+        for (int v = 64 * wv; v < n_vec; v += NT) {
+          const u32x4_t kw = load_vec(v + lane);
+          const int at = 4 * (v + lane);
+          const bool act0 = counted(kw[0], at);
+          const uint64_t am0 = __builtin_amdgcn_ballot_w64(act0);
+          bool meet = false;  // wave-uniform
+          if (am0 != 0u) {
+            const uint32_t bin0 = (kw[0] >> nshift) & mask;
+            const uint32_t b0 =
+                static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(bin0), __builtin_ctzll(am0)));
+            meet = __builtin_popcountll(__builtin_amdgcn_ballot_w64(act0 && bin0 == b0)) >= 16;
           }
-          const uint64_t am = __builtin_amdgcn_ballot_w64(act[e]);
-          if (am == 0u) continue;  // wave-uniform
-          const uint32_t b0 = first_bin(e, am);
-          const uint64_t same = __builtin_amdgcn_ballot_w64(act[e] && bin[e] == b0);
-          if (lane == __builtin_ctzll(am)) atomicAdd(&h[b0], static_cast<uint32_t>(__builtin_popcountll(same)));
-          if (act[e] && bin[e] != b0) atomicAdd(&h[bin[e]], 1u);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if (meet) count_together(kw[e], at + e);
+            else if (counted(kw[e], at + e)) atomicAdd(&h[(kw[e] >> nshift) & mask], 1u);
+          }
+        }
+      } else {
+        // Rows come here because many keys are equal: lanes of a wave mostly meet in one bin.  (The test
+        // above on every step cost 65536 keys of 16 values 12 us of 92.)
+#pragma unroll 1
+        for (int v = 64 * wv; v < n_vec; v += NT) {
+          const u32x4_t kw = load_vec(v + lane);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) count_together(kw[e], 4 * (v + lane) + e);
         }
       }
     }
