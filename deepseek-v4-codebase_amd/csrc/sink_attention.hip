@@ -416,13 +416,25 @@ __global__ __launch_bounds__(kThreads) void hca_compress_rows_kernel(const uint4
   }
 }
 
-// Launches the kernel above when the row's entries fit (at most 4 entries per lane of a wave, else at
-// most 16 per lane of a workgroup), a row has at least two 16-byte pieces per lane of a wave, and the
-// rows' threads fit one launch; false: nothing launched.  Below two pieces, lanes of a row's wave only repeat
-// its last entry, and many rows wait for waves: bf16, 64 columns, general kernel / this one: 8 entries
-// (one piece) 4.0 / 5.4 us for 4096 rows and 26 / 27 for 32768; 16 entries 5.7 / 5.8 and 47 / 28.  32768 rows
-// of one entry of 8 columns: 2.5 / 49 us.  fp32, 64 columns: 4 entries 3.1 / 3.2 and 16 / 13 us, 8 entries 3.9 /
-// 3.4 and 27 / 22.
+// Whether B rows of M entries of ncol 16-byte pieces (of N columns) are the row kernel's.  The general kernel waits
+// M times for memory and reads 2 or 4 bytes per lane; the row kernel spends a wave per row, whose lanes repeat
+// the last entry where M ncol < 64, and reduces over more lanes the fewer the pieces.  So: rows of two pieces per
+// lane, and of 64 pieces an entry; many rows (whose waves queue) when an entry has 32 pieces, or the lanes are
+// mostly used; up to 8192 rows by M^2 ncol, whose line rises with the rows past 1024.  Measured, general / row
+// kernel, bf16: 512 rows of 16 entries x 8 columns 1.03, 12 0.87, 12 x 16 0.96, 8 x 32 0.90, 12 x 32 1.10, 8 x 64 1.06, 6 x
+// 128 1.02, 4 x 256 1.05, 1 x 512 1.05; 2048 of 23 x 8 1.12, 16 x 32 1.06, 12 x 64 1.12, 8 x 64 0.92; 4096 of 32 x 16 1.01, 16 x
+// 64 0.98, 8 x 128 1.05, 1 x 256 1.10; 16384 of 100 x 8 1.87, 64 x 8 0.57, 12 x 64 1.17, 6 x 64 0.69, 3 x 128 0.97; 32768 of
+// 4 x 128 1.31, 1 x 8 0.05.  fp32: 512 of 8 x 8 1.04, 6 x 8 0.96, 4 x 32 1.01, 3 x 64 1.02; 2048 of 12 x 8 1.10, 8 x 8 0.94, 6 x
+// 32 1.10; 4096 of 16 x 16 1.15, 8 x 32 1.02, 6 x 64 1.02; 16384 of 23 x 16 1.47, 16 x 16 0.82.
+bool compress_rows_fit(int64_t B, int64_t M, int64_t ncol, int N) {
+  if (M * ncol >= 128 || ncol >= 64 || (ncol >= 32 && B > 1024)) return true;
+  if (B >= 8192) return M * ncol >= 92 || (B >= 16384 && ncol >= 16 && M >= 3);
+  return M * M * ncol * 1024 >= (N == 8 ? 512 : 128) * std::max<int64_t>(B, 1024);
+}
+
+// Launches the kernel above for the rows it is the faster one for, when their entries fit (at most 4 entries per
+// lane of a wave, else at most 16 per lane of a workgroup) and their threads fit one launch; false: nothing
+// launched.
 template <int DT>
 bool launch_compress_rows(const void* c, const void* z, int64_t B, int64_t M, int64_t D, void* out, hipStream_t st) {
   const int64_t ncol = D * static_cast<int64_t>(dtype_size(DT)) / 16;
@@ -430,7 +442,7 @@ bool launch_compress_rows(const void* c, const void* z, int64_t B, int64_t M, in
       !is_aligned(c, 16) || !is_aligned(z, 16))
     return false;
   const int64_t wave_groups = 64 / ncol, wg_groups = 256 / ncol;
-  if (M < 2 * wave_groups) return false;
+  if (!compress_rows_fit(B, M, ncol, Vec16<DT>::N)) return false;
   const uint4* cv = static_cast<const uint4*>(c);
   const uint4* zv = static_cast<const uint4*>(z);
   auto go = [&](auto fn, int64_t grid) {
@@ -439,7 +451,8 @@ bool launch_compress_rows(const void* c, const void* z, int64_t B, int64_t M, in
                        static_cast<int>(ncol), out);
     return true;
   };
-  if (M == 2 * wave_groups) return go(hca_compress_rows_kernel<DT, 2, 1>, ceil_div(B, int64_t(4)));
+  if (M <= wave_groups) return go(hca_compress_rows_kernel<DT, 1, 1>, ceil_div(B, int64_t(4)));
+  if (M <= 2 * wave_groups) return go(hca_compress_rows_kernel<DT, 2, 1>, ceil_div(B, int64_t(4)));
   if (M <= 4 * wave_groups) return go(hca_compress_rows_kernel<DT, 4, 1>, ceil_div(B, int64_t(4)));
   if (M <= 4 * wg_groups) return go(hca_compress_rows_kernel<DT, 4, 4>, B);
   if (M <= 8 * wg_groups) return go(hca_compress_rows_kernel<DT, 8, 4>, B);

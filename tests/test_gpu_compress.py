@@ -56,14 +56,15 @@ def test_more_rows_than_a_launch_of_whole_waves(dev):
     assert torch.equal(got, c[:, 0])
 
 
-# the line between the kernels: two 16-byte pieces per lane of a wave (128 pieces a row), one entry below and
-# above it, for the narrowest and the widest rows of the row kernel
-@pytest.mark.parametrize("dtype,M,D", [(torch.bfloat16, M, D) for M, D in ((127, 8), (128, 8), (129, 8), (15, 64), (16, 64),
-                                                                         (17, 64), (1, 512), (2, 512), (3, 512))]
-                         + [(torch.float32, M, D) for M, D in ((127, 4), (128, 4), (129, 4), (1, 256), (2, 256), (3, 256))])
-def test_line_between_the_kernels(dev, dtype, M, D):
-    g = torch.Generator().manual_seed(M * D)
-    c, z = torch.randn(5, M, D, generator=g).to(dtype), (torch.randn(5, M, D, generator=g) * 2).to(dtype)
+# the lines between the kernels, below and above them, by rows, entries and columns
+@pytest.mark.parametrize("dtype,B,M,D", [(torch.bfloat16, B, M, D) for B, M, D in (
+    (5, 22, 8), (5, 23, 8), (8192, 91, 8), (8192, 92, 8), (5, 7, 64), (5, 8, 64), (1024, 8, 64), (1025, 8, 64), (2048, 11, 64),
+    (2048, 12, 64), (5, 1, 512), (5, 3, 256), (5, 4, 256), (1025, 1, 256), (16383, 3, 128), (16384, 3, 128), (16384, 2, 128))]
+                         + [(torch.float32, B, M, D) for B, M, D in (
+    (5, 11, 4), (5, 12, 4), (8192, 91, 4), (8192, 92, 4), (2048, 15, 4), (2048, 16, 4), (5, 1, 256), (1025, 1, 128))])
+def test_lines_between_the_kernels(dev, dtype, B, M, D):
+    g = torch.Generator().manual_seed(B + M * D)
+    c, z = torch.randn(B, M, D, generator=g).to(dtype), (torch.randn(B, M, D, generator=g) * 2).to(dtype)
     tol = 1e-5 if dtype == torch.float32 else 5e-3
     np.testing.assert_allclose(to_np_f32(hca_compress(c.to(dev), z.to(dev))), O.hca_compress(to_np_f32(c), to_np_f32(z)),
                                rtol=tol, atol=tol)
